@@ -37,37 +37,6 @@ struct LineMap {
 __device__ inline int last_of_parity(int n, int p) { return (n - 1) - (((n - 1) - p) & 1); }
 
 // ----------------------------------------------------------------- TDMA
-template <typename T>
-__global__ void tdma_solve_kernel(T* __restrict__ u, LineMap g, const double* __restrict__ data,
-                                  int n, int64_t dls, int64_t skip)
-{
-    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nl = g.nlines;
-    if (gid >= 2 * nl) return;
-    const int p = (int)(gid / nl);
-    const int64_t L = gid - (int64_t)p * nl;
-    if (L < skip || p >= n) return;
-    T* v = u + g.off(L);
-    const int64_t sa = g.sa;
-    const double* ld = data + L * dls;
-    const double* d = ld + n;
-    const double* ud = ld + 2 * n + 2;
-    T prev = v[p * sa];
-    for (int i = p + 2; i < n; i += 2) {
-        T cur = sub_mul(v[i * sa], ld[i - 2], prev);
-        v[i * sa] = cur;
-        prev = cur;
-    }
-    const int il = last_of_parity(n, p);
-    T next = divd(v[il * sa], d[il]);
-    v[il * sa] = next;
-    for (int i = il - 2; i >= 0; i -= 2) {
-        T cur = divd(sub_mul(v[i * sa], ud[i], next), d[i]);
-        v[i * sa] = cur;
-        next = cur;
-    }
-}
-
 __global__ void tdma_lu_kernel(double* __restrict__ data, int n, int64_t nbatch)
 {
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -166,19 +135,19 @@ __global__ void pdma_lu_kernel(double* __restrict__ data, int n, int64_t nbatch)
 }
 
 // ----------------------------------------------------------------- DiagMA
+// One thread per element, lanes along the line where the axis is the
+// contiguous one and over lines otherwise.
 template <typename T>
 __global__ void diag_solve_kernel(T* __restrict__ u, LineMap g, const double* __restrict__ dd,
-                                  int n, int64_t dls, int64_t skip)
+                                  int n, int64_t dls, int64_t skip, int along)
 {
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nl = g.nlines;
-    if (gid >= 2 * nl) return;
-    const int p = (int)(gid / nl);
-    const int64_t L = gid - (int64_t)p * nl;
+    if (gid >= g.nlines * n) return;
+    const int64_t L = along ? gid / n : gid % g.nlines;
+    const int i = (int)(along ? gid - L * n : gid / g.nlines);
     if (L < skip) return;
-    T* v = u + g.off(L);
-    const double* d = dd + L * dls;
-    for (int i = p; i < n; i += 2) v[i * g.sa] = divd(v[i * g.sa], d[i]);
+    T* v = u + g.off(L) + (int64_t)i * g.sa;
+    *v = divd(*v, dd[L * dls + i]);
 }
 
 // ----------------------------------------------------------------- other band patterns
@@ -427,143 +396,6 @@ __global__ void helmholtz_lu_kernel(HelmDiags h, const double* __restrict__ alfa
 }
 
 template <typename T>
-__global__ void helmholtz_solve_kernel(const T* __restrict__ b, T* __restrict__ u, LineMap gb,
-                                       LineMap gu, LineMap gf, int M, int neumann,
-                                       const double* __restrict__ d0, const double* __restrict__ d1,
-                                       const double* __restrict__ d2, const double* __restrict__ Lf)
-{
-    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nl = gu.nlines;
-    if (gid >= 2 * nl) return;
-    const int p = (int)(gid / nl);
-    const int64_t L = gid - (int64_t)p * nl;
-    if (p >= M) return;
-    const T* bl = b + gb.off(L);
-    T* ul = u + gu.off(L);
-    const int64_t of = gf.off(L);
-    const int64_t sb = gb.sa, su = gu.sa, sf = gf.sa;
-    // forward elimination, y stored in u
-    T yp = bl[p * sb];
-    ul[p * su] = yp;
-    for (int i = p + 2; i < M; i += 2) {
-        T yv = sub_mul(bl[i * sb], Lf[of + (i - 2) * sf], yp);
-        ul[i * su] = yv;
-        yp = yv;
-    }
-    // back substitution with the running parity sum of the constant tail
-    const int il = last_of_parity(M, p);
-    T n2 = divd(ul[il * su], d0[of + il * sf]);  // u[i+2]
-    ul[il * su] = n2;
-    T n4 = zero<T>();                             // u[i+4]
-    if (il - 2 >= 0) {
-        const int i = il - 2;
-        T cur = divd(sub_mul(ul[i * su], d1[of + i * sf], n2), d0[of + i * sf]);
-        ul[i * su] = cur;
-        n4 = n2;
-        n2 = cur;
-    }
-    T S = zero<T>();
-    for (int i = il - 4; i >= 0; i -= 2) {
-        T cur = sub_mul(ul[i * su], d1[of + i * sf], n2);
-        S = add(S, n4);
-        cur = sub_mul(cur, d2[of + i * sf], S);
-        cur = divd(cur, d0[of + i * sf]);
-        ul[i * su] = cur;
-        n4 = n2;
-        n2 = cur;
-    }
-    if (neumann) {
-        const double d00 = d0[of];
-        if (p == 0 && (d00 - 1.0) * (d00 - 1.0) < 1e-16) ul[0] = zero<T>();
-        for (int i = (p == 0 ? 2 : 1); i < M; i += 2) ul[i * su] = divd(ul[i * su], (double)i * i);
-    }
-}
-
-// Long chains, few lines: one workgroup per (line, parity) chain.  The
-// chain's right-hand side and factors are staged in LDS with coalesced loads
-// (1/d0 formed in parallel there), one thread runs the two sweeps from LDS,
-// and the workgroup stores the result; the thread-per-chain kernel above
-// waits on global memory once per row, which costs milliseconds at N = 4096
-// when there are too few lines to hide it.  Same recurrences
-// (la.pyx:871-912), d0 applied as a multiplication by its reciprocal.
-constexpr int HELM_LDS_MIN_M = 512;
-constexpr int64_t HELM_LDS_MAX_LINES = 2048;
-
-template <typename T>
-__global__ void __launch_bounds__(256)
-    helmholtz_solve_lds_kernel(const T* __restrict__ b, T* __restrict__ u, LineMap gb, LineMap gu,
-                               LineMap gf, int M, int neumann, const double* __restrict__ d0,
-                               const double* __restrict__ d1, const double* __restrict__ d2,
-                               const double* __restrict__ Lf)
-{
-    extern __shared__ __align__(16) unsigned char sm_raw[];
-    const int64_t nl = gu.nlines;
-    const int p = (int)(blockIdx.x / nl);
-    const int64_t L = blockIdx.x - (int64_t)p * nl;
-    const int K = (M - p + 1) / 2;  // rows i = p + 2 m, m < K
-    T* y = reinterpret_cast<T*>(sm_raw);
-    double* Ls = reinterpret_cast<double*>(y + K);
-    double* r0 = Ls + K;
-    double* e1 = r0 + K;
-    double* e2 = e1 + K;
-    const T* bl = b + gb.off(L);
-    T* ul = u + gu.off(L);
-    const int64_t of = gf.off(L);
-    const int64_t sb = gb.sa, su = gu.sa, sf = gf.sa;
-    for (int m = threadIdx.x; m < K; m += blockDim.x) {
-        const int64_t i = p + 2 * m;
-        y[m] = bl[i * sb];
-        Ls[m] = m > 0 ? Lf[of + (i - 2) * sf] : 0.0;
-        r0[m] = 1.0 / d0[of + i * sf];
-        e1[m] = d1[of + i * sf];
-        e2[m] = d2[of + i * sf];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        T yp = y[0];
-#pragma unroll 8
-        for (int m = 1; m < K; ++m) {
-            yp = sub_mul(y[m], Ls[m], yp);
-            y[m] = yp;
-        }
-        T n2 = mul(y[K - 1], r0[K - 1]);
-        y[K - 1] = n2;
-        T n4 = zero<T>();
-        if (K >= 2) {
-            const T cur = mul(sub_mul(y[K - 2], e1[K - 2], n2), r0[K - 2]);
-            y[K - 2] = cur;
-            n4 = n2;
-            n2 = cur;
-        }
-        T S = zero<T>();
-#pragma unroll 8
-        for (int m = K - 3; m >= 0; --m) {
-            T cur = sub_mul(y[m], e1[m], n2);
-            S = add(S, n4);
-            cur = sub_mul(cur, e2[m], S);
-            cur = mul(cur, r0[m]);
-            y[m] = cur;
-            n4 = n2;
-            n2 = cur;
-        }
-    }
-    __syncthreads();
-    for (int m = threadIdx.x; m < K; m += blockDim.x) {
-        const int i = p + 2 * m;
-        T v = y[m];
-        if (neumann) {
-            if (i == 0) {
-                const double d00 = d0[of];
-                if ((d00 - 1.0) * (d00 - 1.0) < 1e-16) v = zero<T>();
-            } else {
-                v = divd(v, (double)i * i);
-            }
-        }
-        ul[(int64_t)i * su] = v;
-    }
-}
-
-template <typename T>
 __global__ void helmholtz_matvec_kernel(const T* __restrict__ v, T* __restrict__ c, LineMap gv,
                                         LineMap gc, int M, int neumann,
                                         const double* __restrict__ A0, const double* __restrict__ At,
@@ -627,6 +459,321 @@ __global__ void poisson_add_kernel(const T* __restrict__ b, T* __restrict__ u, L
         for (int k = p; k < M; k += 2) ul[k * su] = divd(ul[k * su], scale);
 }
 
+// ----------------------------------------------------------------- chain scans
+// TDMA and Helmholtz solves with every chain cut into segments of E rows, one
+// thread each.  A solve is two sweeps of a linear recurrence along the chain
+//   y_m = f_m + a_m y_{m-1}                          (forward elimination)
+//   x_m = f_m + q_m x_{m+1} [+ w_m s_{m+1}],  s_m = s_{m+1} + x_{m+1}
+// (the running sum s is the constant tail of the Chebyshev stiffness rows), so
+// a segment is an affine map of the state that enters it: each thread composes
+// its own, a scan over the segments gives every thread its entering state, and
+// it runs its rows once more.  Bound: a thread per chain waits for memory once
+// per row with too few waves to hide it (8,320 lines of 63 rows at 128^3 are
+// 260 waves on 1,024 SIMDs); here all of a thread's rows are loaded before the
+// first of them is used and a chain is spread over 16 to 256 threads.
+//
+// A workgroup has TL lines x 256 / TL segments, a line's segments TL lanes
+// apart, so that lanes run over lines (coalesced where the lines are
+// neighbours in memory).  Chains longer than 256 / TL * E rows go in chunks,
+// the state carried from one to the next and y kept in u.
+//
+// Measured against a thread per chain (and, for the Helmholtz solve of one long
+// line, a workgroup whose first thread ran both sweeps from LDS): Helmholtz
+// 128 x 128 x 65 complex 47.7 -> 17.4 us (its arrays are 68 MB: 14 us at copy
+// speed), one line of 1024 reals 45.0 -> 5.2 us; TDMA 192 x 96 x 81 complex with
+// shared factors 51.5 -> 17.1 us, 512 x 129 with factors per line, mode 0 in a
+// launch of its own, 194 + 123 -> 7.8 us in one.
+//
+// A segment's factor is kept within +-kChainMax: a product of multipliers that
+// overflowed would turn a line of zeros into NaN, where row by row it stays
+// zero (a state that is not zero overflows either way).
+constexpr double kChainMax = 1e300;
+__device__ inline double chain_clamp(double a) { return fmin(fmax(a, -kChainMax), kChainMax); }
+
+template <typename T>
+struct ChainArgs {
+    const T* b;
+    T* u;
+    LineMap gb, gu;
+    int n;            // rows of the system
+    int64_t skip;     // lines below it are left alone
+    // TDMA: DIA rows of la.pyx:243-252's LU, line L at data + L dls
+    const double* data;
+    int64_t dls;
+    // Helmholtz: factor arrays of LU_Helmholtz (la.pyx:708-843)
+    const double *d0, *d1, *d2, *Lf;
+    LineMap gf;
+    int neumann;
+};
+
+__device__ inline double shflu(double v, int d) { return __shfl_up(v, d); }
+__device__ inline double2 shflu(double2 v, int d) { return make_double2(__shfl_up(v.x, d), __shfl_up(v.y, d)); }
+__device__ inline double shfld(double v, int d) { return __shfl_down(v, d); }
+__device__ inline double2 shfld(double2 v, int d) { return make_double2(__shfl_down(v.x, d), __shfl_down(v.y, d)); }
+__device__ inline double axpb(double a, double x, double b) { return a * x + b; }
+__device__ inline double2 axpb(double a, double2 x, double2 b) { return make_double2(a * x.x + b.x, a * x.y + b.y); }
+
+template <typename T, int TL, int E, bool HELM, bool ONE>
+__global__ void __launch_bounds__(256) chain_solve_kernel(ChainArgs<T> g)
+{
+    constexpr int SG = 256 / TL, WS = 64 / TL, NW = 4;
+    __shared__ double sA[NW][TL];
+    __shared__ T sB[NW][TL];
+    __shared__ double sM[NW][TL][HELM ? 4 : 1];
+    __shared__ T sC[NW][TL][2];
+    const int tid = threadIdx.x, t = tid % TL, seg = tid / TL, wave = tid >> 6, ws = seg % WS;
+    const int p = blockIdx.y, n = g.n;
+    const int64_t L = (int64_t)blockIdx.x * TL + t;
+    const bool valid = L < g.gu.nlines && L >= g.skip;
+    const int64_t Lc = valid ? L : 0;
+    const T* bl = g.b + g.gb.off(Lc);
+    T* ul = g.u + g.gu.off(Lc);
+    const int64_t sb = g.gb.sa, su = g.gu.sa;
+    // lower multiplier of row i at lo[(i - 2) sf], pivot at dg[i sf], upper
+    // bands at up[i sf] and (Helmholtz tail) tl[i sf]
+    const double *lo, *dg, *up, *tl = nullptr;
+    int64_t sf = 1;
+    if constexpr (HELM) {
+        const int64_t of = g.gf.off(Lc);
+        lo = g.Lf + of;
+        dg = g.d0 + of;
+        up = g.d1 + of;
+        tl = g.d2 + of;
+        sf = g.gf.sa;
+    } else {
+        lo = g.data + Lc * g.dls;
+        dg = lo + n;
+        up = lo + 2 * (int64_t)n + 2;
+    }
+    const int K = (n - p + 1) / 2;  // rows i = p + 2 m, m < K
+    const int nch = ONE ? 1 : (K + SG * E - 1) / (SG * E);
+
+    T y[E];
+    double iv[E], q[E], w[HELM ? E : 1];
+    auto load_back = [&](int m0) {  // pivots and upper bands, clamped to row p where outside
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int m = m0 + e;
+            const bool in = valid && m < K, in1 = valid && m + 1 < K;
+            iv[e] = dg[in ? (int64_t)(p + 2 * m) * sf : 0];
+            q[e] = in1 ? up[(int64_t)(p + 2 * m) * sf] : 0.0;
+            if constexpr (HELM) w[e] = valid && m + 2 < K ? tl[(int64_t)(p + 2 * m) * sf] : 0.0;
+        }
+    };
+    // ---------------------------------------------------------- forward
+    T carry = zero<T>();
+    for (int c = 0; c < nch; ++c) {
+        const int m0 = (c * SG + seg) * E;
+        double am[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int m = m0 + e;
+            const bool in = valid && m < K;
+            y[e] = in ? bl[(int64_t)(p + 2 * m) * sb] : zero<T>();
+            am[e] = in && m > 0 ? -lo[(int64_t)(p + 2 * m - 2) * sf] : 0.0;
+        }
+        if (ONE) load_back(m0);
+        double A = 1.0;
+        T B = zero<T>();
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            B = axpb(am[e], B, y[e]);
+            A = chain_clamp(A * am[e]);
+        }
+#pragma unroll
+        for (int k = 1; k < WS; k <<= 1) {
+            const double oA = shflu(A, TL * k);
+            const T oB = shflu(B, TL * k);
+            if (ws >= k) {
+                B = axpb(A, oB, B);
+                A = chain_clamp(A * oA);
+            }
+        }
+        double eA = shflu(A, TL);
+        T eB = shflu(B, TL);
+        if (ws == 0) {
+            eA = 1.0;
+            eB = zero<T>();
+        }
+        if (ws == WS - 1) {
+            sA[wave][t] = A;
+            sB[wave][t] = B;
+        }
+        __syncthreads();
+        T in = carry;
+#pragma unroll
+        for (int k = 0; k < NW; ++k) {
+            carry = axpb(sA[k][t], carry, sB[k][t]);
+            if (k < wave) in = carry;
+        }
+        T yv = axpb(eA, in, eB);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            yv = axpb(am[e], yv, y[e]);
+            y[e] = yv;
+        }
+        if (!ONE) {
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                if (valid && m0 + e < K) ul[(int64_t)(p + 2 * (m0 + e)) * su] = y[e];
+            __syncthreads();  // sA, sB are written again by the next chunk
+        }
+    }
+    // ---------------------------------------------------------- backward
+    T cx = zero<T>(), cs = zero<T>();  // state after the last row
+    for (int c = nch - 1; c >= 0; --c) {
+        const int m0 = (c * SG + seg) * E;
+        if (!ONE) {
+            load_back(m0);
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                y[e] = valid && m0 + e < K ? ul[(int64_t)(p + 2 * (m0 + e)) * su] : zero<T>();
+        }
+        const double d00 = iv[0];
+        T Bx = zero<T>(), Bs = zero<T>();
+        double M00 = 1.0, M01 = 0.0, M10 = 0.0, M11 = 1.0;  // TDMA: M00 alone
+#pragma unroll
+        for (int e = E - 1; e >= 0; --e) {
+            const bool in = valid && m0 + e < K;
+            const double r = 1.0 / iv[e];
+            y[e] = in ? mul(y[e], r) : zero<T>();
+            q[e] = in ? -q[e] * r : 0.0;
+            if constexpr (HELM) {
+                w[e] = in ? -w[e] * r : 0.0;
+                const T nx = add(axpb(q[e], Bx, y[e]), mul(Bs, w[e]));
+                Bs = add(Bs, Bx);
+                Bx = nx;
+                const double n00 = q[e] * M00 + w[e] * M10, n01 = q[e] * M01 + w[e] * M11;
+                M10 += M00;
+                M11 += M01;
+                M00 = n00;
+                M01 = n01;
+            } else {
+                Bx = axpb(q[e], Bx, y[e]);
+                M00 = chain_clamp(M00 * q[e]);
+            }
+        }
+#pragma unroll
+        for (int k = 1; k < WS; k <<= 1) {
+            const double o00 = shfld(M00, TL * k);
+            const T ox = shfld(Bx, TL * k);
+            if constexpr (HELM) {
+                const double o01 = shfld(M01, TL * k), o10 = shfld(M10, TL * k), o11 = shfld(M11, TL * k);
+                const T os = shfld(Bs, TL * k);
+                if (ws + k < WS) {
+                    Bx = add(axpb(M00, ox, Bx), mul(os, M01));
+                    Bs = add(axpb(M10, ox, Bs), mul(os, M11));
+                    const double n00 = M00 * o00 + M01 * o10, n01 = M00 * o01 + M01 * o11;
+                    const double n10 = M10 * o00 + M11 * o10, n11 = M10 * o01 + M11 * o11;
+                    M00 = n00;
+                    M01 = n01;
+                    M10 = n10;
+                    M11 = n11;
+                }
+            } else if (ws + k < WS) {
+                Bx = axpb(M00, ox, Bx);
+                M00 = chain_clamp(M00 * o00);
+            }
+        }
+        // the maps of the segments after this one in the wave
+        double e00 = shfld(M00, TL), e01 = 0.0, e10 = 0.0, e11 = 1.0;
+        T ex = shfld(Bx, TL), es = zero<T>();
+        if constexpr (HELM) {
+            e01 = shfld(M01, TL);
+            e10 = shfld(M10, TL);
+            e11 = shfld(M11, TL);
+            es = shfld(Bs, TL);
+        }
+        if (ws == WS - 1) {
+            e00 = e11 = 1.0;
+            e01 = e10 = 0.0;
+            ex = es = zero<T>();
+        }
+        if (ws == 0) {
+            sM[wave][t][0] = M00;
+            sC[wave][t][0] = Bx;
+            if constexpr (HELM) {
+                sM[wave][t][1] = M01;
+                sM[wave][t][2] = M10;
+                sM[wave][t][3] = M11;
+                sC[wave][t][1] = Bs;
+            }
+        }
+        __syncthreads();
+        T ix = cx, is = cs;
+#pragma unroll
+        for (int k = NW - 1; k >= 0; --k) {
+            if constexpr (HELM) {
+                const T nx = add(axpb(sM[k][t][0], cx, sC[k][t][0]), mul(cs, sM[k][t][1]));
+                cs = add(axpb(sM[k][t][2], cx, sC[k][t][1]), mul(cs, sM[k][t][3]));
+                cx = nx;
+            } else {
+                cx = axpb(sM[k][t][0], cx, sC[k][t][0]);
+            }
+            if (k > wave) {
+                ix = cx;
+                is = cs;
+            }
+        }
+        T x = axpb(e00, ix, ex), s = zero<T>();
+        if constexpr (HELM) {
+            x = add(x, mul(is, e01));
+            s = add(axpb(e10, ix, es), mul(is, e11));
+        }
+#pragma unroll
+        for (int e = E - 1; e >= 0; --e) {
+            const int m = m0 + e, i = p + 2 * m;
+            if constexpr (HELM) {
+                const T nx = add(axpb(q[e], x, y[e]), mul(s, w[e]));
+                s = add(s, x);
+                x = nx;
+            } else {
+                x = axpb(q[e], x, y[e]);
+            }
+            if (valid && m < K) {
+                T out = x;
+                if constexpr (HELM) {
+                    if (g.neumann) {  // column scaling and k = 0 gauge (la.pyx:907-912)
+                        if (i > 0) out = divd(out, (double)i * i);
+                        else if ((d00 - 1.0) * (d00 - 1.0) < 1e-16) out = zero<T>();
+                    }
+                }
+                ul[(int64_t)i * su] = out;
+            }
+        }
+        if (!ONE) __syncthreads();
+    }
+}
+
+template <typename T, int TL, bool HELM>
+static void chain_launch_tl(const ChainArgs<T>& a, hipStream_t s)
+{
+    constexpr int SG = 256 / TL;
+    const int K = (a.n + 1) / 2;
+    const dim3 grid((unsigned)((a.gu.nlines + TL - 1) / TL), 2), block(256);
+    if (K <= SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 1, HELM, true>), grid, block, 0, s, a);
+    else if (K <= 2 * SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 2, HELM, true>), grid, block, 0, s, a);
+    else if (K <= 4 * SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 4, HELM, true>), grid, block, 0, s, a);
+    else if (K <= 8 * SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 8, HELM, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((chain_solve_kernel<T, TL, 8, HELM, false>), grid, block, 0, s, a);
+}
+
+// Lines per workgroup: 16 (256-byte row segments of complex lines) where that
+// still gives every compute unit a workgroup, 2048 lines being 256 of them; else
+// 4, then 1, and as many more segments per chain: below 512 lines of up to 2048
+// rows the arrays are a few MB and latency is the cost, so a chain goes over all
+// 256 threads.  1 also where the axis is the contiguous one (the lanes of a wave
+// then read one line).
+template <typename T, bool HELM>
+static void chain_launch(const ChainArgs<T>& a, hipStream_t s)
+{
+    auto absl = [](int64_t v) { return v < 0 ? -v : v; };
+    const bool across = absl(a.gu.s2) < absl(a.gu.sa) && a.gu.d2 > 1;
+    if (across && a.gu.nlines >= 2048) chain_launch_tl<T, 16, HELM>(a, s);
+    else if (across && a.gu.nlines >= 512) chain_launch_tl<T, 4, HELM>(a, s);
+    else chain_launch_tl<T, 1, HELM>(a, s);
+}
+
 // ----------------------------------------------------------------- host
 static int line_map(int ndim, const int64_t* shape, const int64_t* strides, int axis, LineMap* m,
                     int64_t* n)
@@ -652,6 +799,21 @@ static inline dim3 grid_for(int64_t nthreads, int bs)
 
 using namespace sfa;
 
+template <typename T>
+static ChainArgs<T> tdma_args(T* u, const LineMap& g, const double* data, int64_t n, int64_t dls,
+                              int64_t skip)
+{
+    ChainArgs<T> a{};
+    a.b = u;
+    a.u = u;
+    a.gb = a.gu = g;
+    a.n = (int)n;
+    a.skip = skip;
+    a.data = data;
+    a.dls = dls;
+    return a;
+}
+
 template <int KIND>
 static int banded_solve(void* u, int dtype, int ndim, const int64_t* shape, const int64_t* strides,
                         int axis, const double* data, int64_t n, int64_t dls, int64_t skip,
@@ -668,17 +830,21 @@ static int banded_solve(void* u, int dtype, int ndim, const int64_t* shape, cons
               (long long)n);
     SFA_CHECK(dls >= 0 && skip >= 0, SFA_ERR_ARG, "negative stride/skip");
     const int bs = 256;
-    dim3 grid = grid_for(2 * g.nlines, bs);
+    auto absl = [](int64_t v) { return v < 0 ? -v : v; };
+    const int along = absl(g.sa) <= absl(g.s2) ? 1 : 0;
+    const int64_t nth = KIND == 0 ? g.nlines * n : 2 * g.nlines;
+    SFA_CHECK((nth + bs - 1) / bs < (1ll << 31), SFA_ERR_UNSUPPORTED, "too many lines");
+    dim3 grid = grid_for(nth, bs);
     hipStream_t s = (hipStream_t)stream;
     if (dtype == SFA_C128) {
         double2* uu = (double2*)u;
-        if (KIND == 0) hipLaunchKernelGGL(diag_solve_kernel<double2>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip);
-        if (KIND == 1) hipLaunchKernelGGL(tdma_solve_kernel<double2>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip);
+        if (KIND == 0) hipLaunchKernelGGL(diag_solve_kernel<double2>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip, along);
+        if (KIND == 1) chain_launch<double2, false>(tdma_args(uu, g, data, n, dls, skip), s);
         if (KIND == 2) hipLaunchKernelGGL(pdma_solve_kernel<double2>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip);
     } else {
         double* uu = (double*)u;
-        if (KIND == 0) hipLaunchKernelGGL(diag_solve_kernel<double>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip);
-        if (KIND == 1) hipLaunchKernelGGL(tdma_solve_kernel<double>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip);
+        if (KIND == 0) hipLaunchKernelGGL(diag_solve_kernel<double>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip, along);
+        if (KIND == 1) chain_launch<double, false>(tdma_args(uu, g, data, n, dls, skip), s);
         if (KIND == 2) hipLaunchKernelGGL(pdma_solve_kernel<double>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip);
     }
     SFA_LAUNCH_CHECK();
@@ -853,6 +1019,26 @@ extern "C" int sfa_helmholtz_lu(int neumann, int64_t N, const double* A0, const 
     return SFA_OK;
 }
 
+template <typename T>
+static void helm_launch(const void* b, void* u, const LineMap& gb, const LineMap& gu, const LineMap& gf,
+                        int M, int neumann, const double* d0, const double* d1, const double* d2,
+                        const double* L, hipStream_t s)
+{
+    ChainArgs<T> a{};
+    a.b = (const T*)b;
+    a.u = (T*)u;
+    a.gb = gb;
+    a.gu = gu;
+    a.gf = gf;
+    a.n = M;
+    a.neumann = neumann;
+    a.d0 = d0;
+    a.d1 = d1;
+    a.d2 = d2;
+    a.Lf = L;
+    chain_launch<T, true>(a, s);
+}
+
 extern "C" int sfa_helmholtz_solve(const void* b, void* u, int dtype, int ndim, const int64_t* shape,
                                    const int64_t* b_strides, const int64_t* u_strides, int axis,
                                    int neumann, const double* d0, const double* d1,
@@ -868,33 +1054,10 @@ extern "C" int sfa_helmholtz_solve(const void* b, void* u, int dtype, int ndim, 
     SFA_CHECK(dtype == SFA_F64 || dtype == SFA_C128, SFA_ERR_ARG, "bad dtype %d", dtype);
     SFA_CHECK(N >= 8, SFA_ERR_ARG, "Helmholtz solver needs N >= 8 (got %lld)", (long long)N);
     const int M = (int)N - 2;
-    const size_t elem = dtype == SFA_C128 ? sizeof(double2) : sizeof(double);
-    const size_t lds = (size_t)((M + 1) / 2) * (elem + 4 * sizeof(double));
-    if (M >= HELM_LDS_MIN_M && gu.nlines <= HELM_LDS_MAX_LINES && lds <= 160 * 1024) {
-        dim3 grid((unsigned)(2 * gu.nlines));
-        if (dtype == SFA_C128) {
-            auto k = helmholtz_solve_lds_kernel<double2>;
-            if (lds > 64 * 1024)
-                hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            hipLaunchKernelGGL(k, grid, dim3(256), lds, (hipStream_t)stream, (const double2*)b,
-                               (double2*)u, gb, gu, gf, M, neumann, d0, d1, d2, L);
-        } else {
-            auto k = helmholtz_solve_lds_kernel<double>;
-            if (lds > 64 * 1024)
-                hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            hipLaunchKernelGGL(k, grid, dim3(256), lds, (hipStream_t)stream, (const double*)b,
-                               (double*)u, gb, gu, gf, M, neumann, d0, d1, d2, L);
-        }
-        SFA_LAUNCH_CHECK();
-        return SFA_OK;
-    }
-    dim3 grid = grid_for(2 * gu.nlines, 256);
     if (dtype == SFA_C128)
-        hipLaunchKernelGGL(helmholtz_solve_kernel<double2>, grid, dim3(256), 0, (hipStream_t)stream,
-                           (const double2*)b, (double2*)u, gb, gu, gf, M, neumann, d0, d1, d2, L);
+        helm_launch<double2>(b, u, gb, gu, gf, M, neumann, d0, d1, d2, L, (hipStream_t)stream);
     else
-        hipLaunchKernelGGL(helmholtz_solve_kernel<double>, grid, dim3(256), 0, (hipStream_t)stream,
-                           (const double*)b, (double*)u, gb, gu, gf, M, neumann, d0, d1, d2, L);
+        helm_launch<double>(b, u, gb, gu, gf, M, neumann, d0, d1, d2, L, (hipStream_t)stream);
     SFA_LAUNCH_CHECK();
     return SFA_OK;
 }

@@ -438,12 +438,17 @@ class SolverGeneric1ND:
             b = u
         u = _prepare(b, u)
         data = self.perform_lu(u.device)
-        # mode 0 line: index 0 along every non-axis dim
-        s = [0] * u.dim()
-        s[ax] = slice(None)
-        line0 = u[tuple(s)]
-        self.sol0(line0.unsqueeze(0) if line0.dim() == 0 else line0, axis=0,
-                  constraints=constraints)
+        # mode 0 (index 0 along every non-axis dim) has factors of its own only
+        # where a constraint replaced its first row; the others' launch holds
+        # the same ones otherwise
+        own0 = len(constraints) > 0 or self.sol0._pinned or self._band is not None \
+            or self.kind == "threedma"
+        if own0:
+            s = [0] * u.dim()
+            s[ax] = slice(None)
+            line0 = u[tuple(s)]
+            self.sol0(line0.unsqueeze(0) if line0.dim() == 0 else line0, axis=0,
+                      constraints=constraints)
         shp, st = _geom(u)
         if self._band is not None:
             _lib.call("sfa_band_solve", _lib.ptr(u), _dtype_code(u), u.dim(), shp, st, ax,
@@ -453,9 +458,10 @@ class SolverGeneric1ND:
             _lib.call(self._solve_fn, _lib.ptr(u), _dtype_code(u), u.dim(), shp, st, ax,
                       _lib.ptr(data), self.n, data.shape[1] * data.shape[2], 1, _lib.stream_ptr())
         else:
-            # all modes but the first, one launch (la.py:1346-1364 -> la.pyx:371)
+            # all modes (but the first where it is done), one launch
+            # (la.py:1346-1364 -> la.pyx:371)
             name = {"diag": "DiagMA"}.get(self.kind, self.sol0.__class__.__name__) + "_inner_solve"
-            self.solve_data(u, data, name, ax, True)
+            self.solve_data(u, data, name, ax, own0)
         if self.bc_mats:
             self.bc_mats[0].pmat.space.set_boundary_dofs(u, final=True)
         return u

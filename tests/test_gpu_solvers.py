@@ -266,3 +266,65 @@ def test_solver_generic_matvec_roundtrip(sfa, case):
     G.matvec(ud, c)
     uc = G(c, sfa.Function(T))
     assert rel(uc, ud.cpu().numpy()) < 1e-11
+
+
+@pytest.mark.parametrize("shape,axis", [((3,), 0), ((257, 40, 52), 0), ((261, 2, 1030), 0), ((516, 17, 31), 0),
+                                        ((1030, 130, 4), 0), ((513, 5), 0), ((4105, 3), 0), ((3, 4105), 1),
+                                        ((2, 70, 1100), 1)])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_chain_scan_shapes(sfa, shape, axis, cplx):
+    """The segmented TDMA and Helmholtz solves at the edges of their splits
+    (16, 4 or 1 lines per workgroup; one chunk of rows or several; a chain one
+    row short of, at and beyond a segment boundary), one set of factors and
+    one per line, vs the oracle."""
+    print(f"[chain scan {shape} axis={axis} cplx={cplx}]", flush=True)
+    from shenfun_amd import _lib
+    rng = np.random.default_rng(sum(shape))
+    N = shape[axis]
+    b = rng.standard_normal(shape) + (1j * rng.standard_normal(shape) if cplx else 0.0)
+    d3 = {0: rng.uniform(2, 3, N), -2: rng.uniform(0.1, 1, N - 2), 2: rng.uniform(0.1, 1, N - 2)}
+    lu = S.tdma_lu(S.tdma_dia(d3, N))
+    assert rel(sfa.la.TDMA(sfa.SparseMatrix(d3, (N, N)))(dev(b), axis=axis),
+               S.tdma_solve(b, lu, axis)) < TOL
+    nl = b.size // N
+    if nl <= 2048:  # factors per line, the first line skipped
+        sc = rng.uniform(0.5, 2.0, nl)
+        data = dev(sc[:, None, None] * S.tdma_dia(d3, N)[None])
+        _lib.call("sfa_tdma_lu", _lib.ptr(data), N, nl, _lib.stream_ptr())
+        u = dev(b)
+        _lib.call("sfa_tdma_solve", _lib.ptr(u), _lib.C128 if cplx else _lib.F64, u.dim(),
+                  _lib.arr(u.shape), _lib.arr(u.stride()), axis, _lib.ptr(data), N, 3 * N, 1,
+                  _lib.stream_ptr())
+        ref = np.moveaxis(S.tdma_solve(b, lu, axis), axis, -1).reshape(nl, N) / sc[:, None]
+        ref[0] = np.moveaxis(b, axis, -1).reshape(nl, N)[0]
+        assert rel(np.moveaxis(u.cpu().numpy(), axis, -1).reshape(nl, N), ref) < TOL
+    if N < 8:
+        return
+    ab = [1 if i == axis else n for i, n in enumerate(shape)]
+    beta = rng.uniform(0.5, 50, ab)
+    for bc in ("D", "N"):
+        V = sfa.FunctionSpace(N, "chebyshev", bc=bc)
+        V.axis = axis
+        if len(shape) > 1:
+            class _T:
+                def shape(self, fo=True):
+                    return tuple(shape)
+            V.tensorproductspace = _T()
+        H = sfa.la.Helmholtz(sfa.stiffness_matrix(V), sfa.mass_matrix(V), -np.ones(ab), beta)
+        bd = dev(b)
+        got = H(bd, torch.zeros_like(bd))
+        f = S.helmholtz_lu(bc, N, np.moveaxis(-np.ones(ab), axis, 0)[0], np.moveaxis(beta, axis, 0)[0])
+        ref = np.moveaxis(S.helmholtz_solve(np.moveaxis(b, axis, 0), *f, neumann=(bc == "N")), 0, axis)
+        assert rel(got, ref) < TOL
+        # in place (u = b) the rows of the system are the same
+        assert torch.equal(H(bd).narrow(axis, 0, N - 2), got.narrow(axis, 0, N - 2))
+
+
+def test_chain_scan_zero_lines(sfa):
+    """Lines of zeros stay zero where the product of a chain's multipliers
+    overflows (multipliers above 1 over 1,000 rows), as row by row."""
+    n = 2000
+    d3 = {0: np.full(n, 1.0), -2: np.full(n - 2, 99.0), 2: np.full(n - 2, 1e-4)}
+    b = np.zeros((n, 3))
+    u = sfa.la.TDMA(sfa.SparseMatrix(d3, (n, n)))(dev(b), axis=0)
+    assert torch.equal(u, torch.zeros_like(u))
