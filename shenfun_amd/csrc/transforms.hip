@@ -9,40 +9,9 @@
 // so global accesses coalesce.
 #include <vector>
 
-#include "fft_device.h"
+#include "mix_line.h"
 
 namespace sfa {
-
-// OP_DCT1F / OP_DCT1B: Chebyshev-Gauss-Lobatto scalar product / backward via
-// DCT-I (REDFT00) of length n, computed as the complex FFT of the line's even
-// extension (length 2(n-1)): the sine terms cancel, so the first n outputs
-// are the DCT-I of the real and imaginary parts at once.
-// OP_R2CF / OP_C2RF: odd-length R2C / C2R as a full-length complex FFT (real
-// input widened; Hermitian spectrum completed on load), the even lengths pack
-// pairs of reals instead (OP_R2C / OP_C2R)
-enum LineOp {
-    OP_C2C = 0, OP_R2C = 1, OP_C2R = 2, OP_DCT2 = 3, OP_DCT3 = 4, OP_DCT1F = 5, OP_DCT1B = 6,
-    OP_R2CF = 7, OP_C2RF = 8
-};
-
-struct LineArgs {
-    const char* in;
-    char* out;
-    int64_t in_sa, in_s1, in_s2;
-    int64_t out_sa, out_s1, out_s2;
-    int64_t d1, d2;
-    int n;      // logical length along the axis (real length for R2C/C2R)
-    int ldn;    // LDS line stride (complex elements)
-    int T;      // lines per block
-    int in_cplx, out_cplx;
-    int t_fast_in, t_fast_out;
-    int inv;    // C2C direction
-    double scale;
-    const double* K2;
-    const double2* tw;   // FFT table of length plan.nfft
-    const double2* tw2;  // R2C/C2R: table of length n; DCT: quarter table of length n
-    FFTPlan plan;
-};
 
 __device__ inline double2 ld_elem(const char* base, int64_t off, int cplx)
 {
@@ -351,6 +320,8 @@ static int choose_T(int ldn, int64_t d2)
 
 static int launch_line(int op, bool inv, LineArgs& a, hipStream_t stream)
 {
+    int rc = 0;
+    if (mix_launch(op, inv, a, stream, &rc)) return rc;
     const int ldn = a.ldn;
     const size_t lds = (size_t)2 * a.T * ldn * sizeof(double2) + (size_t)4 * a.T * sizeof(double);
     SFA_CHECK(lds <= 160 * 1024, SFA_ERR_UNSUPPORTED, "transform length %d too large for LDS", a.n);

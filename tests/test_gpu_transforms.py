@@ -291,3 +291,48 @@ def test_project(sfa):
     out = sfa.Function(T)
     assert sfa.project(ch, T, output_array=out, uh_space=C) is out
     assert rel(out, uh.cpu().numpy()) < 1e-12
+
+
+@pytest.mark.parametrize("n", [1, 2, 11, 16, 17, 26, 52, 121, 143, 200, 300, 338, 1001, 2197, 4096, 4100])
+@pytest.mark.parametrize("layout", [0, 1, 2])
+def test_mixed_radix_lines(sfa, n, layout):
+    """Every number of passes and radix of the mixed-radix line kernel (one
+    pass, two to four, a length it refuses), lines interleaved, along the
+    contiguous axis and in tiles that the lines do not fill, in place and out
+    of place: C2C, R2C / C2R (lengths n and 2 n), both Chebyshev quadratures."""
+    print(f"[mixed radix n={n} layout={layout}]", flush=True)
+    m = (5, 21) if n <= 400 else (1, 3)
+    def shp(k):
+        return ((k,) + m, (m[0], k, m[1]), m + (k,))[layout]
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(shp(n)) + 1j * rng.standard_normal(shp(n))
+    B = sfa.FunctionSpace(n, "F", dtype="D")
+    B.axis = layout
+    assert rel(B.scalar_product(dev(x)), np.fft.fft(x, axis=layout) / n) < TOL
+    y = dev(x)
+    B.backward(y, y)
+    assert rel(y, np.fft.ifft(x, axis=layout) * n) < TOL
+    for k in (n, 2 * n):
+        r = rng.standard_normal(shp(k))
+        R = sfa.FunctionSpace(k, "F", dtype="d")
+        R.axis = layout
+        c = np.fft.rfft(r, axis=layout)
+        assert rel(R.scalar_product(dev(r)), c / k) < TOL
+        assert rel(R.backward(dev(c)), r * k) < TOL
+    if n < 3 or n > 4096:
+        return
+    for bc in (None, "D", "N"):
+        for quad in ("GC", "GL") if n <= 2049 else ("GC",):
+            for z in (x, x.real.copy()):
+                V = sfa.FunctionSpace(n, "chebyshev", bc=bc, quad=quad)
+                V.axis = layout
+                ref = S.basis_scalar_product("chebyshev", bc, z, layout, quad=quad)
+                y = dev(z)
+                assert rel(V.scalar_product(y, kind="fast"), ref) < TOL
+                V.scalar_product(y, y, kind="fast")
+                assert rel(y, ref) < TOL
+                if bc is not None:
+                    z = z.copy()
+                    np.moveaxis(z, layout, 0)[n - 2:] = 0
+                assert rel(V.backward(dev(z), kind="fast"),
+                           S.basis_backward("chebyshev", bc, z, layout, quad=quad)) < TOL
