@@ -391,19 +391,27 @@ __device__ __forceinline__ void mix_first(const MixPlan& pl, const MixTile& m, i
                         o = running(o + ss);
                     }
                 } else {
-                    int w0 = twT + nb + j;
+                    // the twiddles in groups of 5: all 15 of a radix 16 at once
+                    // held 60 registers more
+                    int w0 = twT + nb + j, o = buf + j * m.ps + t * m.ts;
+                    lds_put(o, a[0]);
 #pragma unroll
-                    for (int q = 1; q < R; ++q) {
-                        double2 w = lds_get(w0);
-                        w0 = running(w0 + nb);
-                        if (INV) w.y = -w.y;
-                        a[q] = cmul(a[q], w);
-                    }
-                    int o = buf + j * m.ps + t * m.ts;
+                    for (int q0 = 1; q0 < R; q0 += 5) {
+                        double2 w[5];
 #pragma unroll
-                    for (int q = 0; q < R; ++q) {
-                        lds_put(o, a[q]);
-                        o = running(o + step);
+                        for (int i = 0; i < 5; ++i)
+                            if (q0 + i < R) {
+                                w[i] = lds_get(w0);
+                                w0 = running(w0 + nb);
+                            }
+#pragma unroll
+                        for (int i = 0; i < 5; ++i)
+                            if (q0 + i < R) {
+                                if (INV) w[i].y = -w[i].y;
+                                o = running(o + step);
+                                lds_put(o, cmul(a[q0 + i], w[i]));
+                            }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
                 }
             }

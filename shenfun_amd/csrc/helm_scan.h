@@ -304,6 +304,19 @@ __device__ inline void helm_chain_scan(double2* X, int p, int M, double al, doub
 
 namespace sfa {
 
+// 1/d for the LU rows: hardware reciprocal refined by two Newton steps
+// (5 instructions against the IEEE division's scale/fixup sequence; within an
+// ulp for the normal-range pivots here).  The plan builder and the x-pass both
+// regenerate rows through helm_lu_row, so their states agree.
+__device__ inline double helm_rcp(double d)
+{
+    double r = __builtin_amdgcn_rcp(d);
+    double e = __builtin_fma(-d, r, 1.0);
+    r = __builtin_fma(r, e, r);
+    e = __builtin_fma(-d, r, 1.0);
+    return __builtin_fma(r, e, r);
+}
+
 // Row i of (alfa A + beta B) for alfa = -1 from the closed-form Chebyshev
 // SD/SN Galerkin diagonals (chebyshev/matrices.py:221-281, 377-427,
 // 1047-1165), with the Neumann 1/j^2 column scaling and k = 0 gauge row of
@@ -331,30 +344,24 @@ __device__ inline HelmRow helm_row_cf(int i, int M, double be, bool nm, bool zb)
         b0 = hn0 + hp;
         if (i >= 2) bm = -hp;
     } else {
-        const double q = k / (k + 2.0), al = q * q;
-        const double k2i = 1.0 / ((k + 2.0) * (k + 2.0));
-        if (i == 0 && zb) {
-            a0 = -1.0;
-            b0 = 0.0;
+        // columns j scaled by 1/j^2; the scaled entries A_kj / j^2 of a row are
+        // one number, and two reciprocals give all of them
+        const double rk = helm_rcp(i > 0 ? k : 1.0), r2 = helm_rcp(k + 2.0);
+        const double q = k * r2, al = q * q, ii = rk * rk, k2i = r2 * r2;
+        if (i == 0) {
+            a0 = zb ? -1.0 : 0.0;
+            b0 = zb ? 0.0 : hn0;
         } else {
-            a0 = -2.0 * pi * k * k * (k + 1.0) / (k + 2.0);
-            b0 = hn0 + al * al * hp;
-            if (i > 0) {
-                const double ii = 1.0 / (k * k);
-                a0 *= ii;
-                b0 *= ii;
-            }
+            a0 = -2.0 * pi * (k + 1.0) * r2;
+            b0 = (hn0 + al * al * hp) * ii;
         }
+        const double at = -4.0 * pi * (k + 1.0) * k2i;
         if (i < M - 2) {
-            a2 = -4.0 * pi * (k + 2.0) * (k + 2.0) * (k + 1.0) * k2i * k2i;
+            a2 = at;
             b2 = -al * hp * k2i;
         }
-        if (i < M - 4) a4 = -4.0 * pi * (k + 4.0) * (k + 4.0) * (k + 1.0) * k2i / ((k + 4.0) * (k + 4.0));
-        if (i >= 2) {
-            const double qm = (k - 2.0) / k;
-            bm = -(qm * qm) * hp;
-            if (i - 2 >= 1) bm *= 1.0 / ((k - 2.0) * (k - 2.0));
-        }
+        if (i < M - 4) a4 = at;
+        if (i >= 3) bm = -hp * ii;  // (i = 2: the stencil's 0, unscaled)
     }
     r.h = -a0 + be * b0;
     r.s = -a2 + be * b2;
@@ -376,19 +383,6 @@ struct XPlan {
 // form.  State in: (r1, r2, pinv) = (d1/d0, d2/d0, 1/d0) of the previous row of
 // the chain (first = first row of the chain).  Out: this row's 1/d0, the new
 // ratios, and the forward-elimination multiplier am = -L.
-// 1/d for the LU rows: hardware reciprocal refined by two Newton steps
-// (5 instructions against the IEEE division's scale/fixup sequence; within an
-// ulp for the normal-range pivots here).  The plan builder and the x-pass both
-// regenerate rows through helm_lu_row, so their states agree.
-__device__ inline double helm_rcp(double d)
-{
-    double r = __builtin_amdgcn_rcp(d);
-    double e = __builtin_fma(-d, r, 1.0);
-    r = __builtin_fma(r, e, r);
-    e = __builtin_fma(-d, r, 1.0);
-    return __builtin_fma(r, e, r);
-}
-
 __device__ inline void helm_lu_row(const HelmRow& r, int i, int M, bool first, double& r1, double& r2,
                                    double& pinv, double& iv, double& am)
 {

@@ -22,6 +22,7 @@
 
 #include "fft_device.h"
 #include "helm_scan.h"
+#include "xpass_mix.h"
 
 int fft_c2r_add(const void* in, double* out, int ndim, const int64_t* real_shape, const int64_t* in_strides,
                 const int64_t* out_strides, int axis, double scale, void* stream, const double* add,
@@ -275,6 +276,16 @@ struct PlanLayout {
     int64_t nl, nu, K, E, off_s, off_bs, bytes;
 };
 
+// Rows per segment for chains of at most K rows: the next size that the
+// x-pass kernels are built for (beyond 16: no such kernel, any size will do).
+static int64_t segment_rows(int64_t K)
+{
+    const int64_t e = (K + 15) / 16;
+    for (int64_t v : {1, 2, 3, 4, 6, 8, 12, 16})
+        if (e <= v) return v;
+    return e;
+}
+
 static int64_t round256(int64_t b) { return (b + 255) / 256 * 256; }
 
 static void plan_shape(int64_t Nx, int64_t Ny, int64_t Nz, PlanLayout* L, std::vector<int>* map,
@@ -283,7 +294,7 @@ static void plan_shape(int64_t Nx, int64_t Ny, int64_t Nz, PlanLayout* L, std::v
     const int64_t Nzh = Nz / 2 + 1;
     L->nl = Ny * Nzh;
     L->K = (Nx - 2 + 1) / 2;
-    L->E = (L->K + 15) / 16;
+    L->E = segment_rows(L->K);
     std::vector<int64_t> sv((size_t)L->nl);
     for (int64_t j = 0; j < Ny; ++j) {
         const int64_t ky = (j < Ny / 2 || (Ny % 2 == 1 && j == Ny / 2)) ? j : j - Ny;
@@ -398,6 +409,48 @@ static const double* plan_lift(const void* plan)
     return it == g_plans.end() ? nullptr : it->second.lift;
 }
 
+// The x-pass on the plan's restart states for lengths with prime factors up to
+// 13; false where the length does not allow it.
+static bool xpass_mix(double2* W, int Nx, int Ny, int Nzh, int Kp, double alpha, int neumann, const double* K2,
+                      const XPlan& pv, int64_t nb, hipStream_t s, int* rc)
+{
+    XMixArgs a;
+    const int64_t E = segment_rows((Nx - 2 + 1) / 2);
+    if (E > 16 || nb > 65535 || !make_mix_plan(Nx, true, &a.plan)) return false;
+    a.W = W;
+    a.sa = (int64_t)Ny * Kp;
+    a.bstride = (int64_t)Nx * a.sa;
+    a.nl = a.sa;
+    if (a.nl >= (1ll << 31)) return false;
+    a.Kp = Kp;
+    a.Nzh = Nzh;
+    a.N = Nx;
+    const int nat = (Nx - 1) + (Nx - 1) / (2 * (int)E) + 1;  // natural order, padded
+    a.LS = (nat > a.plan.size() ? nat : a.plan.size()) | 1;  // odd: lines in distinct banks
+    if (xpass_mix_lds(a) > 160 * 1024) return false;
+    a.neumann = neumann;
+    a.alpha = alpha;
+    a.K2 = K2;
+    a.pl = pv;
+    a.tw = fft_table(Nx);
+    a.tq = quarter_table(Nx);
+    if (!a.tw || !a.tq) {
+        *rc = fail(SFA_ERR_HIP, "table allocation failed");
+        return true;
+    }
+    switch (E) {
+        case 1: *rc = xpass_mix_1(a, nb, s); break;
+        case 2: *rc = xpass_mix_2(a, nb, s); break;
+        case 3: *rc = xpass_mix_3(a, nb, s); break;
+        case 4: *rc = xpass_mix_4(a, nb, s); break;
+        case 6: *rc = xpass_mix_6(a, nb, s); break;
+        case 8: *rc = xpass_mix_8(a, nb, s); break;
+        case 12: *rc = xpass_mix_12(a, nb, s); break;
+        default: *rc = xpass_mix_16(a, nb, s); break;
+    }
+    return true;
+}
+
 // W: nb arrays (Nx, Ny, Nzh) of complex lines at kz pitch Kp >= Nzh, back to back.
 int xpass_launch(double2* W, int Nx, int Ny, int Nzh, int Kp, double alpha, int neumann,
                  hipStream_t s, const void* plan, int64_t nb)
@@ -410,6 +463,7 @@ int xpass_launch(double2* W, int Nx, int Ny, int Nzh, int Kp, double alpha, int 
                   "plan does not match the solve");
         int rc = 0;
         if (fast_xpass(W, Nx, Ny, Nzh, Kp, alpha, neumann, K2, pv, nb, s, &rc)) return rc;
+        if (xpass_mix(W, Nx, Ny, Nzh, Kp, alpha, neumann, K2, pv, nb, s, &rc)) return rc;
     }
     if (nb > 1) {  // the generic kernel takes one array per launch
         for (int64_t b = 0; b < nb; ++b) {
@@ -638,7 +692,7 @@ extern "C" int sfa_helmholtz3d_plan(int64_t Nx, int64_t Ny, int64_t Nz, double a
     if (rc) return rc;
     PlanLayout L = head.L;
     L.K = (Nx - 2 + 1) / 2;
-    L.E = (L.K + 15) / 16;
+    L.E = segment_rows(L.K);
     SFA_CHECK(plan_bytes >= L.bytes, SFA_ERR_ARG, "plan buffer too small (%lld < %lld)",
               (long long)plan_bytes, (long long)L.bytes);
     hipStream_t s = (hipStream_t)stream;

@@ -84,6 +84,21 @@ def test_helmholtz3d_fused_repeat_identical(sfa):
     assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("bc,alpha", [("D", 0.0), ("N", 0.0), ("N", 2.0)])
+@pytest.mark.parametrize("Nx", [8, 9, 16, 33, 35, 66, 98, 99, 130, 132, 182, 195, 250, 260, 384, 390, 507])
+def test_helmholtz3d_xpass_lengths(sfa, Nx, bc, alpha):
+    """The fused x-pass on every segment size (1, 2, 3, 4, 6, 8, 12, 16 rows,
+    lengths at both ends of each), odd lengths and a last workgroup of two
+    lines, vs the oracle; alpha = 0 with Neumann ends is the gauge."""
+    print(f"[xpass Nx={Nx} {bc} alpha={alpha}]", flush=True)
+    f = S.helmholtz3d_rhs(Nx, 6, 4, seed=Nx)
+    T = sfa.TensorProductSpace(None, (sfa.FunctionSpace(Nx, "chebyshev", bc=bc),
+                                      sfa.FunctionSpace(6, "F", dtype="D"),
+                                      sfa.FunctionSpace(4, "F", dtype="d")))
+    u = sfa.HelmholtzSolver3D(T, alpha)(dev(f))
+    assert rel(u, S.helmholtz3d_cheb_fourier(f, alpha, bc)[0]) < 1e-12
+
+
 @pytest.mark.parametrize("precision,shape,bc", [("fp64", (32, 24, 16), "D"), ("fp64", (64, 20, 16), "N"),
                                                ("fp64", (64, 16, 128), "D"), ("mixed", (64, 32, 64), "D"),
                                                ("mixed", (128, 16, 64), "N")])
