@@ -184,6 +184,16 @@ int sfa_line_matmul(const void* in, void* out, int dtype, int ndim,
                     const int64_t* out_strides, int axis, int64_t nout,
                     const double* M, void* stream);
 
+/* sfa_line_matmul for a matrix of even and odd functions on symmetric nodes:
+ * parity 1, the rows are the functions, M[k][nin-1-j] = (-1)^k M[k][j]
+ * (analysis); parity 2, the columns, M[nout-1-j][k] = (-1)^k M[j][k]
+ * (synthesis).  The matrix-product form then reads one half of M and does half
+ * the products on the even and odd parts. */
+int sfa_line_matmul_parity(const void* in, void* out, int dtype, int ndim,
+                           const int64_t* in_shape, const int64_t* in_strides,
+                           const int64_t* out_strides, int axis, int64_t nout, const double* M,
+                           int parity, void* stream);
+
 /* Evaluation of a 1-3D expansion at scattered points: out[p] = sum over
  * (k0, k1, k2) of c[k0][k1][k2] E0[p][k0] E1[p][k1] E2[p][k2]; E_d device
  * complex128 (npts, n_d), each axis' basis functions at the points'

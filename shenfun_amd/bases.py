@@ -324,12 +324,22 @@ class _PolyBase(SpectralBase):
             return _lib.F64
         raise TypeError(f"unsupported dtype {t.dtype} (float64 / complex128 only)")
 
-    # dense per-line contraction: 'recursive' / 'vandermonde' kinds
-    def _matmul(self, inp, out, M):
+    # phi_k(-x) = (-1)^k phi_k(x): the orthogonal polynomials and the stencils
+    # of offsets 0, 2, 4
+    _even_odd = True
+
+    # dense per-line contraction: 'recursive' / 'vandermonde' kinds.  parity: 1
+    # if M's rows are the basis functions (analysis), 2 if its columns are
+    # (synthesis), on the family's symmetric nodes
+    def _matmul(self, inp, out, M, parity):
         shp, sin = _geom(inp)
         _, sout = _geom(out)
-        _lib.call("sfa_line_matmul", _lib.ptr(inp), _lib.ptr(out), self._dtype_code(inp), inp.dim(),
-                  shp, sin, sout, self.axis, int(M.shape[0]), _lib.ptr(M), _lib.stream_ptr())
+        args = (_lib.ptr(inp), _lib.ptr(out), self._dtype_code(inp), inp.dim(), shp, sin, sout,
+                self.axis, int(M.shape[0]), _lib.ptr(M))
+        if self._even_odd:
+            _lib.call("sfa_line_matmul_parity", *args, parity, _lib.stream_ptr())
+        else:
+            _lib.call("sfa_line_matmul", *args, _lib.stream_ptr())
         return out
 
     def _analysis_matrix(self):
@@ -697,7 +707,7 @@ class ChebyshevBase(_PolyBase):
         else:
             if out.data_ptr() == inp.data_ptr():
                 raise ValueError("dense transform cannot run in place")
-            self._matmul(inp, out, self._analysis_matrix())
+            self._matmul(inp, out, self._analysis_matrix(), 1)
 
     def _backward(self, inp, out, kind):
         kind = self._auto(kind, inp, out)
@@ -708,7 +718,7 @@ class ChebyshevBase(_PolyBase):
             _lib.call(fn, _lib.ptr(inp), _lib.ptr(out), self._dtype_code(inp),
                       inp.dim(), shp, sin, sout, self.axis, _lib.ptr(self._K2()), _lib.stream_ptr())
         else:
-            self._matmul(inp, out, self._synthesis_matrix())
+            self._matmul(inp, out, self._synthesis_matrix(), 2)
 
 
 class LegendreBase(_PolyBase):
@@ -756,10 +766,10 @@ class LegendreBase(_PolyBase):
     def _scalar_product(self, inp, out, kind):
         if out.data_ptr() == inp.data_ptr():
             raise ValueError("Legendre transforms cannot run in place")
-        self._matmul(inp, out, self._analysis_matrix())
+        self._matmul(inp, out, self._analysis_matrix(), 1)
 
     def _backward(self, inp, out, kind):
-        self._matmul(inp, out, self._synthesis_matrix())
+        self._matmul(inp, out, self._synthesis_matrix(), 2)
 
 
 def _legendre_pd(n, x):
@@ -1164,6 +1174,10 @@ class _StencilSpace:
     def bc_kind(self):
         return self.kind
 
+    @property
+    def _even_odd(self):
+        return self.kind not in ("DN", "ND")  # their stencils have an offset 1
+
     def dim(self):
         return self.N - self._nbc[self.kind]
 
@@ -1195,10 +1209,10 @@ class _StencilSpace:
     def _scalar_product(self, inp, out, kind):
         if out.data_ptr() == inp.data_ptr():
             raise ValueError("dense transform cannot run in place")
-        self._matmul(inp, out, self._analysis_matrix())
+        self._matmul(inp, out, self._analysis_matrix(), 1)
 
     def _backward(self, inp, out, kind):
-        self._matmul(inp, out, self._synthesis_matrix())
+        self._matmul(inp, out, self._synthesis_matrix(), 2)
 
     def forward(self, input_array=None, output_array=None, kind=None):
         if self.kind in ("DN", "ND"):

@@ -43,21 +43,39 @@ struct B2Prob {
 // ----------------------------------------------------------------- MFMA GEMM
 constexpr int B2_THREADS = GEMM_THREADS;
 
-// C (m x n, ldc) = A (m x k, lda) B (k x n, ldb), all row-major FP64, by the
-// whole workgroup (4 waves in a 2 x 2 grid over BM x BN block tiles, K in
-// steps of BK).  sA: BK x (BM + 1) doubles, sB: BK x BN doubles of LDS.
-// Out-of-range operand elements load as zero; stores are bounds-checked.
-// Each output is one MFMA accumulation chain over K in ascending steps of 4
-// (up to the last step holding k), so the result does not depend on BM, BN,
+// The stage's product (fold_tile: all four matrices are even and odd functions
+// on symmetric grids) by the whole workgroup, in tiles of BM x BN outputs, K
+// folded and in steps of BK.  An output's MFMA chain does not depend on BM, BN,
 // BK, on which workgroup computes the tile, or on the order of the tiles.
-template <int BM, int BN, int BK>
-__device__ void block_gemm(const double* __restrict__ A, int64_t lda, const double* __restrict__ B,
-                           int64_t ldb, double* __restrict__ C, int64_t ldc, int m, int n, int k,
-                           double* sA, double* sB)
+template <int MODE>
+constexpr int b2_bmu(int BM) { return MODE == FOLD_ROWS_IN || MODE == FOLD_ROWS_OUT ? BM / 2 : BM; }
+template <int MODE>
+constexpr int b2_bnu(int BN) { return MODE == FOLD_ROWS_IN || MODE == FOLD_ROWS_OUT ? BN : BN / 2; }
+
+template <int MODE, int BM, int BN, int BK>
+__device__ __forceinline__ void block_gemm(const double* __restrict__ A, int64_t lda, const double* __restrict__ B,
+                                           int64_t ldb, double* __restrict__ C, int64_t ldc, int m, int n, int k,
+                                           double* sm)
 {
-    for (int m0 = 0; m0 < m; m0 += BM)
-        for (int n0 = 0; n0 < n; n0 += BN) gemm_tile<BM, BN, BK>(A, lda, B, ldb, C, ldc, m, n, k, m0, n0, sA, sB);
+    constexpr bool rows = MODE == FOLD_ROWS_IN || MODE == FOLD_ROWS_OUT;
+    const int mu = rows ? (m + 1) / 2 : m;
+    const int nu = rows ? n : (MODE == FOLD_COLS_IN ? n / 2 : n / 2 + 1);
+    for (int m0 = 0; m0 < mu; m0 += b2_bmu<MODE>(BM))
+        for (int n0 = 0; n0 < nu; n0 += b2_bnu<MODE>(BN))
+            fold_tile<MODE, b2_bmu<MODE>(BM), b2_bnu<MODE>(BN), BK>(A, lda, B, ldb, C, ldc, m, n, k, m0, n0, sm,
+                                                                     sm + FoldShape<b2_bmu<MODE>(BM), b2_bnu<MODE>(BN)>::template lds_a<BK>());
     __syncthreads();  // C complete and LDS free before the caller's next stage
+}
+
+// LDS doubles of a tile over the modes
+template <int BM, int BN, int BK>
+constexpr int b2_lds()
+{
+    using R = FoldShape<BM / 2, BN>;
+    using C = FoldShape<BM, BN / 2>;
+    constexpr int rows = R::template lds_a<BK>() + R::template lds_b<BK>();
+    constexpr int cols = C::template lds_a<BK>() + C::template lds_b<BK>();
+    return rows > cols ? rows : cols;
 }
 
 // ----------------------------------------------------------------- per-ky solve
@@ -206,8 +224,7 @@ struct B2Args {
 template <int BM, int BN, int BK>
 __global__ void __launch_bounds__(B2_THREADS) batch2d_kernel(B2Args a)
 {
-    __shared__ double sA[BK * (BM + 1)];
-    __shared__ double sB[BK * BN];
+    __shared__ double sm[b2_lds<BM, BN, BK>()];
     const int b = blockIdx.x;
     double* W0 = a.work + (int64_t)b * a.wstride;
     for (int q = a.blk_ptr[b]; q < a.blk_ptr[b + 1]; ++q) {
@@ -220,28 +237,16 @@ __global__ void __launch_bounds__(B2_THREADS) batch2d_kernel(B2Args a)
         const double* P = a.mats + pr.p_off;
         const double* Df = a.mats + pr.df_off;
         const double* Di = a.mats + pr.di_off;
-        // The four contractions through one GEMM call site (a loop over the
-        // stages, not unrolled): with four inlined copies the compiler held the
-        // address setup of all of them, 163 VGPRs against 67 for one tile.
-#pragma unroll 1
-        for (int st = 0; st < 4; ++st) {
-            const double *A, *B;
-            double* C;
-            int64_t lda, ldb, ldc;
-            int m, n, k;
-            if (st == 0) {  // T1 = P f (M x Ny), held in u
-                A = P, lda = Nx, B = f, ldb = Ny, C = u, ldc = Ny, m = M, n = Ny, k = Nx;
-            } else if (st == 1) {  // T2 = T1 Df (M x L) in W0
-                A = u, lda = Ny, B = Df, ldb = L, C = W0, ldc = L, m = M, n = L, k = Ny;
-            } else if (st == 2) {  // U1 = Phi u_hat (Nx x L) in W1
-                // per-ky solve in place first, W1 as the Thomas scratch
-                batch_solve(W0, L, M, Nyh, pr.bc, pr.alpha, W1);
-                A = Phi, lda = M, B = W0, ldb = L, C = W1, ldc = L, m = Nx, n = L, k = M;
-            } else {  // u = U1 Di (Nx x Ny)
-                A = W1, lda = L, B = Di, ldb = Ny, C = u, ldc = Ny, m = Nx, n = Ny, k = L;
-            }
-            block_gemm<BM, BN, BK>(A, lda, B, ldb, C, ldc, m, n, k, sA, sB);
-        }
+        // T1 = P f (M x Ny), held in u
+        block_gemm<FOLD_ROWS_IN, BM, BN, BK>(P, Nx, f, Ny, u, Ny, M, Ny, Nx, sm);
+        // T2 = T1 Df (M x L) in W0
+        block_gemm<FOLD_COLS_IN, BM, BN, BK>(u, Ny, Df, L, W0, L, M, L, Ny, sm);
+        // per-ky solve in place, W1 as the Thomas scratch
+        batch_solve(W0, L, M, Nyh, pr.bc, pr.alpha, W1);
+        // U1 = Phi u_hat (Nx x L) in W1
+        block_gemm<FOLD_ROWS_OUT, BM, BN, BK>(Phi, M, W0, L, W1, L, Nx, L, M, sm);
+        // u = U1 Di (Nx x Ny)
+        block_gemm<FOLD_COLS_OUT, BM, BN, BK>(W1, L, Di, Ny, u, Ny, Nx, Ny, L, sm);
     }
 }
 
@@ -252,7 +257,7 @@ __global__ void __launch_bounds__(B2_THREADS) batch2d_kernel(B2Args a)
 // Per-problem intermediates live at work + woff[p] (W0: (Nx-2) x (Ny+2),
 // then W1: Nx x (Ny+2)); T1 is held in u as in the persistent kernel.
 struct B2Task {
-    int32_t prob, m0, n0, tile;  // tile: 0 = 32 x 32, 1 = 64 x 64 block tile
+    int32_t prob, m0, n0, tile;  // first unit row and column of the tile; tile class
 };
 
 struct B2WideArgs {
@@ -267,28 +272,10 @@ struct B2WideArgs {
 };
 
 constexpr int B2W_BK = 16;
-// block tiles of the tile classes (a 128 x 64 class spills in this kernel)
+// output tiles (rows, columns) of the tile classes, by stage parity: the
+// contractions over x (stages 0, 2) fold rows, those over y (1, 3) columns
 constexpr int kB2WClasses = 2;
-constexpr int kB2WTile[kB2WClasses][2] = {{32, 32}, {64, 64}};
-
-template <int BM, int BN>
-__device__ void wide_gemm(const B2WideArgs& a, const B2Task& tk, int stage, double* sA, double* sB)
-{
-    const B2Prob pr = a.probs[tk.prob];
-    const int Nx = pr.Nx, Ny = pr.Ny, M = Nx - 2, L = Ny + 2;
-    double* u = a.U + pr.u_off;
-    double* W0 = a.work + a.woff[tk.prob];
-    double* W1 = W0 + (int64_t)M * L;
-    if (stage == 0)  // T1 = P f (M x Ny) in u
-        gemm_tile<BM, BN, B2W_BK>(a.mats + pr.p_off, Nx, a.F + pr.f_off, Ny, u, Ny, M, Ny, Nx, tk.m0, tk.n0,
-                                  sA, sB);
-    else if (stage == 1)  // T2 = T1 Df (M x L) in W0
-        gemm_tile<BM, BN, B2W_BK>(u, Ny, a.mats + pr.df_off, L, W0, L, M, L, Ny, tk.m0, tk.n0, sA, sB);
-    else if (stage == 2)  // U1 = Phi u_hat (Nx x L) in W1
-        gemm_tile<BM, BN, B2W_BK>(a.mats + pr.phi_off, M, W0, L, W1, L, Nx, L, M, tk.m0, tk.n0, sA, sB);
-    else  // u = U1 Di (Nx x Ny)
-        gemm_tile<BM, BN, B2W_BK>(W1, L, a.mats + pr.di_off, Ny, u, Ny, Nx, Ny, L, tk.m0, tk.n0, sA, sB);
-}
+constexpr int kB2WTile[kB2WClasses][2][2] = {{{32, 64}, {64, 32}}, {{64, 64}, {64, 64}}};
 
 // One task per workgroup, all of a launch's tasks of tile class CLS; every
 // output keeps its one MFMA chain over K, so the results do not depend on the
@@ -296,10 +283,41 @@ __device__ void wide_gemm(const B2WideArgs& a, const B2Task& tk, int stage, doub
 template <int STAGE, int CLS>
 __global__ void __launch_bounds__(B2_THREADS) batch2d_tile_kernel(B2WideArgs a)
 {
-    constexpr int BM = kB2WTile[CLS][0], BN = kB2WTile[CLS][1];
-    __shared__ double sA[B2W_BK * (BM + 1)];
-    __shared__ double sB[B2W_BK * BN];
-    wide_gemm<BM, BN>(a, a.tasks[blockIdx.x], STAGE, sA, sB);
+    constexpr int MODE = STAGE == 0 ? FOLD_ROWS_IN : STAGE == 1 ? FOLD_COLS_IN : STAGE == 2 ? FOLD_ROWS_OUT : FOLD_COLS_OUT;
+    constexpr int BMU = b2_bmu<MODE>(kB2WTile[CLS][STAGE & 1][0]), BNU = b2_bnu<MODE>(kB2WTile[CLS][STAGE & 1][1]);
+    __shared__ double sA[FoldShape<BMU, BNU>::template lds_a<B2W_BK>()];
+    __shared__ double sB[FoldShape<BMU, BNU>::template lds_b<B2W_BK>()];
+    const B2Task tk = a.tasks[blockIdx.x];
+    const B2Prob pr = a.probs[tk.prob];
+    const int Nx = pr.Nx, Ny = pr.Ny, M = Nx - 2, L = Ny + 2;
+    double* u = a.U + pr.u_off;
+    double* W0 = a.work + a.woff[tk.prob];
+    double* W1 = W0 + (int64_t)M * L;
+    if constexpr (STAGE == 0)  // T1 = P f (M x Ny) in u
+        fold_tile<MODE, BMU, BNU, B2W_BK>(a.mats + pr.p_off, Nx, a.F + pr.f_off, Ny, u, Ny, M, Ny, Nx, tk.m0, tk.n0,
+                                          sA, sB);
+    else if constexpr (STAGE == 1)  // T2 = T1 Df (M x L) in W0
+        fold_tile<MODE, BMU, BNU, B2W_BK>(u, Ny, a.mats + pr.df_off, L, W0, L, M, L, Ny, tk.m0, tk.n0, sA, sB);
+    else if constexpr (STAGE == 2)  // U1 = Phi u_hat (Nx x L) in W1
+        fold_tile<MODE, BMU, BNU, B2W_BK>(a.mats + pr.phi_off, M, W0, L, W1, L, Nx, L, M, tk.m0, tk.n0, sA, sB);
+    else  // u = U1 Di (Nx x Ny)
+        fold_tile<MODE, BMU, BNU, B2W_BK>(W1, L, a.mats + pr.di_off, Ny, u, Ny, Nx, Ny, L, tk.m0, tk.n0, sA, sB);
+}
+
+// Unit rows and columns of a stage's product, and of its tiles.
+struct B2Units {
+    int64_t m, n, bm, bn;
+};
+static B2Units b2_units(int st, int cls, int64_t Nx, int64_t Ny)
+{
+    const int64_t M = Nx - 2, L = Ny + 2;
+    const int64_t bm = kB2WTile[cls][st & 1][0], bn = kB2WTile[cls][st & 1][1];
+    switch (st) {
+        case 0: return {(M + 1) / 2, Ny, bm / 2, bn};
+        case 1: return {M, L / 2, bm, bn / 2};
+        case 2: return {(Nx + 1) / 2, L, bm / 2, bn};
+        default: return {Nx, Ny / 2 + 1, bm, bn / 2};
+    }
 }
 
 template <int STAGE>
@@ -665,10 +683,11 @@ static void b2_wide_shape(int nprob, const int* Nx, const int* Ny, int64_t ntask
     int64_t cnt[4][kB2WClasses] = {};
     for (int i = 0; i < nprob; ++i) {
         const int64_t M = Nx[i] - 2, L = Ny[i] + 2, X = Nx[i], Y = Ny[i];
-        const int64_t mm[4] = {M, M, X, X}, nn[4] = {Y, L, L, Y};
         for (int st = 0; st < 4; ++st)
-            for (int c = 0; c < kB2WClasses; ++c)
-                cnt[st][c] += cdiv(mm[st], kB2WTile[c][0]) * cdiv(nn[st], kB2WTile[c][1]);
+            for (int c = 0; c < kB2WClasses; ++c) {
+                const B2Units t = b2_units(st, c, X, Y);
+                cnt[st][c] += cdiv(t.m, t.bm) * cdiv(t.n, t.bn);
+            }
         *work += (M * L + X * L + 31) / 32 * 32;
     }
     for (int st = 0; st < 4; ++st) {
@@ -676,6 +695,50 @@ static void b2_wide_shape(int nprob, const int* Nx, const int* Ny, int64_t ntask
         while (c > 0 && cnt[st][c] < 4 * kWideCus) --c;
         ntask[st] = cnt[st][c];
         if (cls) cls[st] = c;
+    }
+}
+
+// A stage's tasks in launch order.  Workgroups go to the 8 XCDs in turn, so the
+// tiles of a problem, which share its operands, take every eighth place and read
+// them through one L2 (in the order of the problems most of the eight fetched
+// them: 1,024 problems up to 512 x 256, the four stages 719 -> 631 us; they were
+// 1,011 before the contractions were folded).  The tasks with the longest K come
+// first.  A problem with more than a 64th of the tasks is cut into runs of that
+// many, so that few problems still use every XCD.
+static void b2_wide_order(int st, int cls, int nprob, const int* Nx, const int* Ny, int64_t ntask,
+                          std::vector<B2Task>& out)
+{
+    std::vector<int> ids(nprob);
+    std::iota(ids.begin(), ids.end(), 0);
+    auto klen = [&](int i) { return st % 2 == 0 ? Nx[i] : Ny[i]; };
+    std::stable_sort(ids.begin(), ids.end(), [&](int a, int b) { return klen(a) > klen(b); });
+    const int64_t run = std::max<int64_t>(4, ntask / 64);
+    std::vector<B2Task> q[8];
+    double load[8] = {};
+    for (int i : ids) {
+        const B2Units t = b2_units(st, cls, Nx[i], Ny[i]);
+        const double cost = klen(i) / 32.0 + 4.0;  // K steps of 16 units, and a tile's start and end
+        int64_t left = 0;
+        int x = 0;
+        for (int m0 = 0; m0 < t.m; m0 += (int)t.bm)
+            for (int n0 = 0; n0 < t.n; n0 += (int)t.bn) {
+                if (left-- == 0) {
+                    left = run - 1;
+                    x = (int)(std::min_element(load, load + 8) - load);
+                }
+                q[x].push_back(B2Task{i, m0, n0, cls});
+                load[x] += cost;
+            }
+    }
+    size_t at[8] = {};
+    out.clear();
+    out.reserve((size_t)ntask);
+    for (int64_t n = 0; n < ntask; ++n) {
+        int x = (int)(n % 8);
+        if (at[x] == q[x].size())  // this XCD's list is done: from the longest rest
+            for (int y = 0; y < 8; ++y)
+                if (q[y].size() - at[y] > q[x].size() - at[x]) x = y;
+        out.push_back(q[x][at[x]++]);
     }
 }
 
@@ -904,16 +967,11 @@ extern "C" int sfa_batch2d_wide_plan(int nprob, const int* Nx, const int* Ny, co
     wi.off_probs = 0;
     wi.mats = mats;
     std::vector<B2Task> tasks[4];
+    for (int st = 0; st < 4; ++st) b2_wide_order(st, cls[st], nprob, Nx, Ny, wi.ntask[st], tasks[st]);
     std::vector<int64_t> woff(nprob);
     int64_t w = 0;
     for (int i = 0; i < nprob; ++i) {
-        const int M = Nx[i] - 2, L = Ny[i] + 2, X = Nx[i], Y = Ny[i];
-        const int mm[4] = {M, M, X, X}, nn[4] = {Y, L, L, Y};
-        for (int st = 0; st < 4; ++st) {
-            const int bm = kB2WTile[cls[st]][0], bn = kB2WTile[cls[st]][1];
-            for (int m0 = 0; m0 < mm[st]; m0 += bm)
-                for (int n0 = 0; n0 < nn[st]; n0 += bn) tasks[st].push_back(B2Task{i, m0, n0, cls[st]});
-        }
+        const int M = Nx[i] - 2, L = Ny[i] + 2, X = Nx[i];
         woff[i] = w;
         w += ((int64_t)M * L + (int64_t)X * L + 31) / 32 * 32;
     }

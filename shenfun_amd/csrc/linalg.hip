@@ -232,10 +232,55 @@ __global__ void __launch_bounds__(GEMM_THREADS)
     line_gemm_kernel(const double* __restrict__ M, const double* __restrict__ X, double* __restrict__ Y,
                      int nout, int nin, int64_t ncol, int64_t ldx, int64_t ldy)
 {
-    __shared__ double sA[16 * (64 + 1)];
-    __shared__ double sB[16 * 64];
+    __shared__ double sA[16 * (64 + 8)];
+    __shared__ double sB[16 * (64 + 8)];
     gemm_tile<64, 64, 16>(M, nin, X, ldx, Y, ldy, nout, (int)ncol, nin,
                           (int)blockIdx.y * 64, (int)blockIdx.x * 64, sA, sB);
+}
+
+// Workgroup id -> column tile x < nx and row tile y < ny.  Workgroups go to the
+// 8 XCDs in turn: the ny row tiles of a column tile get ids 8 apart, so that
+// they read its data through one L2 at about the same time.
+__device__ inline void xcd_tile(int id, int nx, int ny, int& x, int& y)
+{
+    const int g = id / (8 * ny), r = id - g * 8 * ny;
+    const int w = nx - 8 * g < 8 ? nx - 8 * g : 8;
+    y = r / w;
+    x = 8 * g + r - y * w;
+}
+
+// The same with M even and odd functions on symmetric nodes: half the products
+// (fold_tile), and half of M read.  Tiles of 64 x 64 outputs, 32 x 64 where those
+// are fewer than the compute units (on 16640 columns at 128 x 128 the smaller
+// tiles read the data twice as often: 32 us against 16).  Against the plain form,
+// microseconds: 128 x 128 on 16640 columns 22.3 -> 16 (a copy of in and out: 7),
+// 512 x 512 on 258 35.9 -> 17, 64 x 64 on 66 6.9 -> 5.3; the two larger ones are
+// bound by their few workgroups (260 and 80), a chain of 4 to 16 K steps each.
+template <int MODE, int BMU, int BNU, int BK>
+__global__ void __launch_bounds__(GEMM_THREADS)
+    line_gemm_fold_kernel(const double* __restrict__ M, const double* __restrict__ X, double* __restrict__ Y,
+                          int nout, int nin, int64_t ncol, int64_t ldx, int64_t ldy)
+{
+    using Sh = FoldShape<BMU, BNU>;
+    __shared__ double sA[Sh::template lds_a<BK>()];
+    __shared__ double sB[Sh::template lds_b<BK>()];
+    int x, y;
+    xcd_tile((int)blockIdx.x, (int)((ncol + BNU - 1) / BNU), ((nout + 1) / 2 + BMU - 1) / BMU, x, y);
+    fold_tile<MODE, BMU, BNU, BK>(M, nin, X, ldx, Y, ldy, nout, (int)ncol, nin, y * BMU, x * BNU, sA, sB);
+}
+
+template <int MODE>
+static void line_gemm_fold(const double* M, const double* X, double* Y, int nout, int nin, int64_t ncol,
+                           int64_t ldx, int64_t ldy, hipStream_t s)
+{
+    const int mu = (nout + 1) / 2;
+    const int64_t nx = (ncol + 63) / 64;
+    if (nx * ((mu + 31) / 32) >= 256)
+        hipLaunchKernelGGL((line_gemm_fold_kernel<MODE, 32, 64, 16>), dim3((unsigned)(nx * ((mu + 31) / 32))),
+                           dim3(GEMM_THREADS), 0, s, M, X, Y, nout, nin, ncol, ldx, ldy);
+    else
+        hipLaunchKernelGGL((line_gemm_fold_kernel<MODE, 16, 64, 16>), dim3((unsigned)(nx * ((mu + 15) / 16))),
+                           dim3(GEMM_THREADS), 0, s, M, X, Y, nout, nin, ncol, ldx, ldy);
 }
 
 }  // namespace sfa
@@ -274,10 +319,9 @@ extern "C" int sfa_recursion_matrix(const double* x, const double* w, int64_t Nx
     return SFA_OK;
 }
 
-extern "C" int sfa_line_matmul(const void* in, void* out, int dtype, int ndim,
-                               const int64_t* in_shape, const int64_t* in_strides,
-                               const int64_t* out_strides, int axis, int64_t nout, const double* M,
-                               void* stream)
+static int line_matmul(const void* in, void* out, int dtype, int ndim, const int64_t* in_shape,
+                       const int64_t* in_strides, const int64_t* out_strides, int axis, int64_t nout,
+                       const double* M, int parity, void* stream)
 {
     Geom gi, go;
     int rc;
@@ -297,6 +341,13 @@ extern "C" int sfa_line_matmul(const void* in, void* out, int dtype, int ndim,
     if (nlines > 16 && flat(gi) && flat(go) && nlines * (dtype == SFA_C128 ? 2 : 1) <= INT32_MAX) {
         const int w = dtype == SFA_C128 ? 2 : 1;  // doubles per element
         const int64_t ncol = nlines * w;
+        if (parity) {
+            auto run = parity == 1 ? line_gemm_fold<FOLD_ROWS_IN> : line_gemm_fold<FOLD_ROWS_OUT>;
+            run(M, (const double*)in, (double*)out, (int)nout, (int)gi.n, ncol, gi.sa * w, go.sa * w,
+                (hipStream_t)stream);
+            SFA_LAUNCH_CHECK();
+            return SFA_OK;
+        }
         dim3 g((unsigned)((ncol + 63) / 64), (unsigned)((nout + 63) / 64));
         hipLaunchKernelGGL(line_gemm_kernel, g, dim3(GEMM_THREADS), 0, (hipStream_t)stream, M,
                            (const double*)in, (double*)out, (int)nout, (int)gi.n, ncol, gi.sa * w,
@@ -328,6 +379,23 @@ extern "C" int sfa_line_matmul(const void* in, void* out, int dtype, int ndim,
                            gi.s2, go.sa, go.s1, go.s2, gi.d2, nlines, tfi, tfo);
     SFA_LAUNCH_CHECK();
     return SFA_OK;
+}
+
+extern "C" int sfa_line_matmul(const void* in, void* out, int dtype, int ndim,
+                               const int64_t* in_shape, const int64_t* in_strides,
+                               const int64_t* out_strides, int axis, int64_t nout, const double* M,
+                               void* stream)
+{
+    return line_matmul(in, out, dtype, ndim, in_shape, in_strides, out_strides, axis, nout, M, 0, stream);
+}
+
+extern "C" int sfa_line_matmul_parity(const void* in, void* out, int dtype, int ndim,
+                                      const int64_t* in_shape, const int64_t* in_strides,
+                                      const int64_t* out_strides, int axis, int64_t nout, const double* M,
+                                      int parity, void* stream)
+{
+    SFA_CHECK(parity == 1 || parity == 2, SFA_ERR_ARG, "line_matmul: parity must be 1 (rows) or 2 (columns)");
+    return line_matmul(in, out, dtype, ndim, in_shape, in_strides, out_strides, axis, nout, M, parity, stream);
 }
 
 // ----------------------------------------------------------------- point evaluation

@@ -336,3 +336,29 @@ def test_mixed_radix_lines(sfa, n, layout):
                     np.moveaxis(z, layout, 0)[n - 2:] = 0
                 assert rel(V.backward(dev(z), kind="fast"),
                            S.basis_backward("chebyshev", bc, z, layout, quad=quad)) < TOL
+
+
+@pytest.mark.parametrize("parity", [1, 2])
+@pytest.mark.parametrize("nout,nin,lines", [(8, 8, 17), (9, 9, 33), (31, 32, 40), (33, 31, 17), (64, 64, 32), (65, 64, 33),
+                                            (130, 128, 300), (512, 512, 65), (64, 66, 5000), (7, 130, 5000), (64, 64, 5),
+                                            (1, 1, 20), (2, 3, 20)])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_line_matmul_parity(sfa, parity, nout, nin, lines, cplx):
+    """sfa_line_matmul_parity on matrices of even and odd functions vs the full
+    product: odd and even lengths on both sides, tile edges, both tile sizes,
+    a length below one K step, and few lines (the row-parallel form)."""
+    print(f"[line_matmul_parity {parity} {nout}x{nin} lines={lines} cplx={cplx}]", flush=True)
+    from shenfun_amd import _lib
+    rng = np.random.default_rng(nout + nin + lines)
+    M = rng.standard_normal((nout, nin))
+    if parity == 1:
+        M = M + (-1.0) ** np.arange(nout)[:, None] * M[:, ::-1]
+    else:
+        M = M + (-1.0) ** np.arange(nin)[None, :] * M[::-1]
+    X = rng.standard_normal((nin, lines)) + (1j * rng.standard_normal((nin, lines)) if cplx else 0.0)
+    x, m = dev(X), dev(M)
+    y = torch.full((nout, lines), np.nan, dtype=x.dtype, device="cuda")
+    _lib.call("sfa_line_matmul_parity", _lib.ptr(x), _lib.ptr(y), _lib.C128 if cplx else _lib.F64, 2,
+              _lib.arr(X.shape), _lib.arr(x.stride()), _lib.arr(y.stride()), 0, nout, _lib.ptr(m), parity,
+              _lib.stream_ptr())
+    assert rel(y, M @ X) < 1e-13
