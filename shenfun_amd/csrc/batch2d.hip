@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "common.h"
+#include "helm_scan.h"
 #include "mfma_gemm.h"
 
 namespace sfa {
@@ -67,7 +68,9 @@ __device__ __forceinline__ void block_gemm(const double* __restrict__ A, int64_t
     __syncthreads();  // C complete and LDS free before the caller's next stage
 }
 
-// LDS doubles of a tile over the modes
+constexpr int kB2SolveLds = 6 * 2 * 2 * 8;  // doubles of LDS of the per-ky solves
+
+// LDS doubles of a tile over the modes, and of the solves
 template <int BM, int BN, int BK>
 constexpr int b2_lds()
 {
@@ -75,7 +78,8 @@ constexpr int b2_lds()
     using C = FoldShape<BM, BN / 2>;
     constexpr int rows = R::template lds_a<BK>() + R::template lds_b<BK>();
     constexpr int cols = C::template lds_a<BK>() + C::template lds_b<BK>();
-    return rows > cols ? rows : cols;
+    constexpr int tile = rows > cols ? rows : cols;
+    return tile > kB2SolveLds ? tile : kB2SolveLds;
 }
 
 // ----------------------------------------------------------------- per-ky solve
@@ -83,129 +87,252 @@ constexpr int b2_lds()
 // h_k = 2/(2k+1):  SD  A_kk = 4k+6, B_kk = h_k + h_{k+2}, B_{k,k+2} = -h_{k+2};
 // SN  a_k = k(k+1)/((k+2)(k+3)), A_kk = h_k a_k (k+1/2)((k+2)(k+3) - k(k+1)),
 //     B_kk = h_k + a_k^2 h_{k+2}, B_{k,k+2} = -a_k h_{k+2}.  B is symmetric.
+// Reciprocals by helm_rcp (5 instructions, within an ulp).
 __device__ inline void leg_rows(int i, int bc, double& Akk, double& Bkk, double& Bup)
 {
     const double k = (double)i;
-    const double h0 = 2.0 / (2.0 * k + 1.0), h2 = 2.0 / (2.0 * k + 5.0);
+    const double h0 = 2.0 * helm_rcp(2.0 * k + 1.0), h2 = 2.0 * helm_rcp(2.0 * k + 5.0);
     if (bc == 0) {
         Akk = 4.0 * k + 6.0;
         Bkk = h0 + h2;
         Bup = -h2;
     } else {
-        const double a = k * (k + 1.0) / ((k + 2.0) * (k + 3.0));
+        const double a = k * (k + 1.0) * helm_rcp((k + 2.0) * (k + 3.0));
         Akk = h0 * a * (k + 0.5) * ((k + 2.0) * (k + 3.0) - k * (k + 1.0));
         Bkk = h0 + a * a * h2;
         Bup = -a * h2;
     }
 }
 
-// Thomas algorithm per (ky, parity chain) on the complex columns of W0 (M rows,
-// row pitch ldw doubles, column ky at 2 ky).  cp: scratch, M * Nyh doubles,
-// row-major (row i, column ky), so a wave's stores of one step are contiguous
-// (ky-major, a chain's own column, they were 32 separate lines per wave: the
-// solve launch of the tile-parallel form took 1.21 ms instead of 0.83 ms for
-// the 4096-problem batch).  Staging row chunks in LDS between barriers measured
-// slower still (1.43 ms).  Neumann with beta = 0 (ky = 0, alpha = 0): the singular row 0
-// is replaced by u_0 = 0 (the constraint (0, 0) of the reference's mode-0
-// solver).
-// One row of the forward elimination (the reference's TDMA order), x = (re, im)
-// of row i in, its reduced values out.
-__device__ __forceinline__ void thomas_row(int i, int M, int bc, double beta, double2& x, double& cc,
-                                           double& cprev, double& rprev_re, double& rprev_im,
-                                           double& lprev_up)
-{
-    double Akk, Bkk, Bup;
-    leg_rows(i, bc, Akk, Bkk, Bup);
-    const double d = Akk + beta * Bkk;
-    const double up = (i + 2 < M) ? beta * Bup : 0.0;
-    const double lo = (i >= 2) ? lprev_up : 0.0;  // B symmetric: B_{i,i-2} = B_{i-2,i}
-    double rr_re, rr_im;
-    if (bc == 1 && i == 0 && fabs(beta) < 1e-12) {
-        cc = 0.0;
-        rr_re = rr_im = 0.0;
-    } else {
-        const double dd = 1.0 / (d - lo * cprev);
-        cc = up * dd;
-        rr_re = (x.x - lo * rprev_re) * dd;
-        rr_im = (x.y - lo * rprev_im) * dd;
+// Rows i, i + 2, .. of A + beta B (M rows): diagonal d, upper up, lower lo (=
+// the upper one of row i - 2).  Neumann with beta = 0 (ky = 0, alpha = 0): the
+// singular row 0 is replaced by u_0 = 0 (the constraint (0, 0) of the
+// reference's mode-0 solver), told by gauge.
+struct LegRows {
+    double d, up, lo, bup;
+    bool gauge;
+    __device__ __forceinline__ LegRows(int i, int bc)
+    {
+        double x0, x1;
+        bup = 0.0;
+        if (i >= 2) leg_rows(i - 2, bc, x0, x1, bup);
     }
-    x = make_double2(rr_re, rr_im);
-    cprev = cc;
-    rprev_re = rr_re;
-    rprev_im = rr_im;
-    lprev_up = up;
+    __device__ __forceinline__ void row(int i, int M, int bc, double beta)
+    {
+        lo = beta * bup;
+        double Akk, Bkk;
+        leg_rows(i, bc, Akk, Bkk, bup);
+        d = Akk + beta * Bkk;
+        up = i + 2 < M ? beta * bup : 0.0;
+        gauge = bc == 1 && i == 0 && fabs(beta) < 1e-12;
+    }
+};
+
+// The per-ky solves of TL neighbouring columns (c0 ..) of W0 (M rows, row pitch
+// ldw doubles, column ky at 2 ky complex), in place, by the whole workgroup:
+// every (ky, parity) chain is cut into 128 / TL segments of E rows, one thread
+// each, which reads its rows once and holds them through the three recurrences
+// of the Thomas algorithm,
+//   c_i = up_i / (d_i - lo_i c_{i-2})            a Moebius map of c
+//   r_i = (x_i - lo_i r_{i-2}) / (d_i - ..)      affine in r
+//   u_i = r_i - c_i u_{i+2}                      affine in u
+// For each, a thread composes its segment's map, a scan over the segments (lanes
+// TL apart of one wave, then the parity's two waves through LDS) gives it the
+// state that enters, and it runs its rows again.  Bound by the array's one read and one
+// write; a thread per chain made four passes over it and two over a pivot
+// scratch: 1,024 problems up to 512 x 256, 221 us -> 117 us.
+template <int E, int TL>
+__device__ __forceinline__ void leg_solve_group(double* __restrict__ W0, int64_t ldw, int M, int Nyh, int c0, int bc,
+                                                double alpha, double* sm)
+{
+    constexpr int WS = 64 / TL;  // segments of a wave
+    const int tid = threadIdx.x;
+    const int t = tid % TL, seg = (tid & 127) / TL, p = tid >> 7, ws = seg % WS, w1 = (tid >> 6) & 1;
+    const int ky = c0 + t;
+    const bool valid = ky < Nyh;
+    const double beta = alpha + (double)ky * (double)ky;
+    // the first row, opaque to the optimiser for each of the two passes that form
+    // the rows: it kept the first pass' rows for the second one (and, in the
+    // persistent kernel, for the next columns), three numbers a row in registers
+    int m0 = seg * E;
+    asm volatile("" : "+v"(m0));
+    const int K = (M - p + 1) / 2;
+    double2* xc = reinterpret_cast<double2*>(W0 + 2 * (valid ? ky : 0)) + (int64_t)p * (ldw / 2);
+    // number c of wave w of this parity, line t
+    auto slot = [&](int c, int w) -> double& { return sm[((c * 2 + w) * 2 + p) * TL + t]; };
+    double2 x[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int m = m0 + e < K ? m0 + e : K - 1;  // (beyond the chain: read again, replaced below)
+        x[e] = xc[(int64_t)m * ldw];
+    }
+    // 1. the segment's map of c as a 2 x 2 matrix on (numerator, denominator)
+    double n0 = 1.0, n1 = 0.0, e0 = 0.0, e1 = 1.0;
+    auto scaled = [&]() {  // by a power of two, the largest entry in [1/2, 1)
+        const double mx = fmax(fmax(fabs(n0), fabs(n1)), fmax(fabs(e0), fabs(e1)));
+        const int ex = -__builtin_amdgcn_frexp_exp(mx);
+        n0 = ldexp(n0, ex);
+        n1 = ldexp(n1, ex);
+        e0 = ldexp(e0, ex);
+        e1 = ldexp(e1, ex);
+    };
+    {
+        LegRows r(p + 2 * m0, bc);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            if (m0 + e < K) {
+                r.row(p + 2 * (m0 + e), M, bc, beta);
+                const double u = r.gauge ? 0.0 : r.up, d = r.gauge ? 1.0 : r.d, l = r.gauge ? 0.0 : r.lo;
+                const double a0 = u * e0, a1 = u * e1;
+                e0 = d * e0 - l * n0;
+                e1 = d * e1 - l * n1;
+                n0 = a0;
+                n1 = a1;
+            }
+            if (e % 4 == 3 || e == E - 1) scaled();
+        }
+    }
+#pragma unroll
+    for (int k = 1; k < WS; k <<= 1) {  // (this segment's map) o (the earlier ones')
+        const double on0 = __shfl_up(n0, TL * k), on1 = __shfl_up(n1, TL * k);
+        const double oe0 = __shfl_up(e0, TL * k), oe1 = __shfl_up(e1, TL * k);
+        if (ws >= k) {
+            const double a0 = n0 * on0 + n1 * oe0, a1 = n0 * on1 + n1 * oe1;
+            const double b0 = e0 * on0 + e1 * oe0, b1 = e0 * on1 + e1 * oe1;
+            n0 = a0;
+            n1 = a1;
+            e0 = b0;
+            e1 = b1;
+            scaled();
+        }
+    }
+    if (ws == WS - 1) {  // c = 0 before the chain: the image of (0, 1)
+        slot(0, w1) = n1;
+        slot(1, w1) = e1;
+    }
+    double pn0 = __shfl_up(n0, TL), pn1 = __shfl_up(n1, TL), pe0 = __shfl_up(e0, TL), pe1 = __shfl_up(e1, TL);
+    if (ws == 0) {
+        pn0 = pe1 = 1.0;
+        pn1 = pe0 = 0.0;
+    }
+    __syncthreads();
+    const double num0 = w1 ? slot(0, 0) : 0.0, den0 = w1 ? slot(1, 0) : 1.0;
+    const double num = pn0 * num0 + pn1 * den0, den = pe0 * num0 + pe1 * den0;
+    // 2. the rows' pivots from there, and the segment's map of r
+    asm volatile("" : "+v"(m0));
+    double cc = num * helm_rcp(den);
+    double cu[E], al[E];
+    double A = 1.0;
+    double2 B = make_double2(0.0, 0.0);
+    {
+        LegRows r(p + 2 * m0, bc);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            cu[e] = al[e] = 0.0;
+            if (m0 + e < K) {
+                r.row(p + 2 * (m0 + e), M, bc, beta);
+                const double dd = r.gauge ? 0.0 : helm_rcp(r.d - r.lo * cc);
+                cc = r.up * dd;
+                cu[e] = cc;
+                al[e] = -r.lo * dd;
+                x[e] = make_double2(x[e].x * dd, x[e].y * dd);
+            } else {
+                x[e] = make_double2(0.0, 0.0);
+            }
+            B = make_double2(al[e] * B.x + x[e].x, al[e] * B.y + x[e].y);
+            A *= al[e];
+        }
+    }
+#pragma unroll
+    for (int k = 1; k < WS; k <<= 1) {
+        const double oA = __shfl_up(A, TL * k), ox = __shfl_up(B.x, TL * k), oy = __shfl_up(B.y, TL * k);
+        if (ws >= k) {
+            B = make_double2(A * ox + B.x, A * oy + B.y);
+            A *= oA;
+        }
+    }
+    if (ws == WS - 1) {
+        slot(2, w1) = B.x;
+        slot(3, w1) = B.y;
+    }
+    double pA = __shfl_up(A, TL);
+    double2 pB = make_double2(__shfl_up(B.x, TL), __shfl_up(B.y, TL));
+    if (ws == 0) {
+        pA = 1.0;
+        pB = make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+    double2 v = w1 ? make_double2(slot(2, 0), slot(3, 0)) : make_double2(0.0, 0.0);
+    v = make_double2(pA * v.x + pB.x, pA * v.y + pB.y);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        v = make_double2(al[e] * v.x + x[e].x, al[e] * v.y + x[e].y);
+        if (m0 + e < K) x[e] = v;  // (beyond the chain r and c stay 0: the state there)
+    }
+    // 3. back substitution
+    A = 1.0;
+    B = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int e = E - 1; e >= 0; --e) {
+        B = make_double2(x[e].x - cu[e] * B.x, x[e].y - cu[e] * B.y);
+        A *= -cu[e];
+    }
+#pragma unroll
+    for (int k = 1; k < WS; k <<= 1) {
+        const double oA = __shfl_down(A, TL * k), ox = __shfl_down(B.x, TL * k), oy = __shfl_down(B.y, TL * k);
+        if (ws + k < WS) {
+            B = make_double2(A * ox + B.x, A * oy + B.y);
+            A *= oA;
+        }
+    }
+    if (ws == 0) {
+        slot(4, w1) = B.x;
+        slot(5, w1) = B.y;
+    }
+    pA = __shfl_down(A, TL);
+    pB = make_double2(__shfl_down(B.x, TL), __shfl_down(B.y, TL));
+    if (ws == WS - 1) {
+        pA = 1.0;
+        pB = make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+    v = w1 ? make_double2(0.0, 0.0) : make_double2(slot(4, 1), slot(5, 1));
+    v = make_double2(pA * v.x + pB.x, pA * v.y + pB.y);
+#pragma unroll
+    for (int e = E - 1; e >= 0; --e) {
+        v = make_double2(x[e].x - cu[e] * v.x, x[e].y - cu[e] * v.y);
+        if (valid && m0 + e < K) xc[(int64_t)(m0 + e) * ldw] = v;
+    }
 }
 
-__device__ __forceinline__ void batch_solve(double* __restrict__ W0, int64_t ldw, int M, int Nyh, int bc,
-                                            double alpha, double* __restrict__ cp)
+// Columns per group of the solves of chains of K rows: with 128 / TL segments
+// of at most 8 rows.
+__host__ __device__ inline int leg_solve_tl(int K) { return K <= 128 ? 8 : K <= 256 ? 4 : 2; }
+
+// The solves of the column groups first, first + step, .. of a problem.  Rows
+// per segment by the chain's length alone, so that a column's arithmetic does
+// not depend on how the problem is launched.
+__device__ __forceinline__ void batch_solve(double* __restrict__ W0, int64_t ldw, int M, int Nyh, int bc, double alpha,
+                                            int first, int step, double* sm)
 {
-    // A chain's row loads do not depend on its recurrence: the sweeps take the
-    // rows D at a time from one of two register buffers while the next D rows
-    // load into the other, so a step does not wait out a load of its own
-    // (clamped row indices keep the loads unconditional).
-    constexpr int D = 8;
-    for (int c = threadIdx.x; c < 2 * Nyh; c += blockDim.x) {
-        const int ky = c >> 1, p = c & 1;
-        const double beta = alpha + (double)ky * (double)ky;
-        double* cpc = cp + ky;  // cpc[i * Nyh]
-        double2* xc = reinterpret_cast<double2*>(W0 + 2 * ky);  // row i at xc[i * ldw / 2]
-        const int64_t lx = ldw / 2;
-        double cprev = 0.0, rprev_re = 0.0, rprev_im = 0.0, lprev_up = 0.0;
-        int last = -1;
-        double2 bA[D], bB[D];
-        auto fwd = [&](int i0, double2 (&cur)[D], double2 (&nxt)[D]) {
-#pragma unroll
-            for (int d = 0; d < D; ++d) nxt[d] = xc[min(i0 + 2 * (D + d), M - 1) * lx];
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const int i = i0 + 2 * d;
-                if (i < M) {
-                    double cc;
-                    thomas_row(i, M, bc, beta, cur[d], cc, cprev, rprev_re, rprev_im, lprev_up);
-                    cpc[(int64_t)i * Nyh] = cc;
-                    xc[i * lx] = cur[d];
-                    last = i;
-                }
-            }
-        };
-#pragma unroll
-        for (int d = 0; d < D; ++d) bA[d] = xc[min(p + 2 * d, M - 1) * lx];
-        for (int i0 = p; i0 < M; i0 += 4 * D) {
-            fwd(i0, bA, bB);
-            if (i0 + 2 * D < M) fwd(i0 + 2 * D, bB, bA);
+    const int K = (M + 1) / 2;
+    auto run = [&](auto Ec, auto Tc) {
+        constexpr int E = decltype(Ec)::value, TL = decltype(Tc)::value;
+        for (int c0 = first * TL; c0 < Nyh; c0 += step * TL) {
+            leg_solve_group<E, TL>(W0, ldw, M, Nyh, c0, bc, alpha, sm);
+            __syncthreads();  // the columns' LDS maps are read
         }
-        // back substitution over the same rows, last to first
-        double xr = 0.0, xi = 0.0;
-        double2 cA[D], cB[D];
-        double kA[D], kB[D];
-        auto bwd = [&](int i0, double2 (&cx)[D], double (&ck)[D], double2 (&nx)[D], double (&nk)[D]) {
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const int i = max(i0 - 2 * (D + d), 0);
-                nx[d] = xc[i * lx];
-                nk[d] = cpc[(int64_t)i * Nyh];
-            }
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const int i = i0 - 2 * d;
-                if (i >= 0) {
-                    xr = cx[d].x - ck[d] * xr;
-                    xi = cx[d].y - ck[d] * xi;
-                    xc[i * lx] = make_double2(xr, xi);
-                }
-            }
-        };
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            const int i = max(last - 2 * d, 0);
-            cA[d] = xc[i * lx];
-            kA[d] = cpc[(int64_t)i * Nyh];
-        }
-        for (int i0 = last; i0 >= 0; i0 -= 4 * D) {
-            bwd(i0, cA, kA, cB, kB);
-            if (i0 - 2 * D >= 0) bwd(i0 - 2 * D, cB, kB, cA, kA);
-        }
-    }
+    };
+    using T8 = std::integral_constant<int, 8>;
+    using T4 = std::integral_constant<int, 4>;
+    using T2 = std::integral_constant<int, 2>;
+    if (K <= 32) run(T2{}, T8{});
+    else if (K <= 64) run(T4{}, T8{});
+    else if (K <= 96) run(std::integral_constant<int, 6>{}, T8{});
+    else if (K <= 128) run(T8{}, T8{});
+    else if (K <= 192) run(std::integral_constant<int, 6>{}, T4{});
+    else if (K <= 256) run(T8{}, T4{});
+    else run(T8{}, T2{});
     __syncthreads();
 }
 
@@ -241,8 +368,8 @@ __global__ void __launch_bounds__(B2_THREADS) batch2d_kernel(B2Args a)
         block_gemm<FOLD_ROWS_IN, BM, BN, BK>(P, Nx, f, Ny, u, Ny, M, Ny, Nx, sm);
         // T2 = T1 Df (M x L) in W0
         block_gemm<FOLD_COLS_IN, BM, BN, BK>(u, Ny, Df, L, W0, L, M, L, Ny, sm);
-        // per-ky solve in place, W1 as the Thomas scratch
-        batch_solve(W0, L, M, Nyh, pr.bc, pr.alpha, W1);
+        // per-ky solve in place
+        batch_solve(W0, L, M, Nyh, pr.bc, pr.alpha, 0, 1, sm);
         // U1 = Phi u_hat (Nx x L) in W1
         block_gemm<FOLD_ROWS_OUT, BM, BN, BK>(Phi, M, W0, L, W1, L, Nx, L, M, sm);
         // u = U1 Di (Nx x Ny)
@@ -266,7 +393,7 @@ struct B2WideArgs {
     const B2Prob* probs;
     const B2Task* tasks;   // this stage's tasks
     const int64_t* woff;   // per problem, in doubles
-    const int* order;      // the solve launch's problem per workgroup
+    const int2* groups;    // the solve launch's problem and column group per workgroup
     const double* mats;
     double* work;
 };
@@ -334,11 +461,10 @@ static int launch_wide_stage(const B2WideArgs& a, int cls, int64_t ntask, hipStr
 
 __global__ void __launch_bounds__(B2_THREADS) batch2d_wide_solve_kernel(B2WideArgs a)
 {
-    const int p = a.order[blockIdx.x];
-    const B2Prob pr = a.probs[p];
-    const int Nx = pr.Nx, Ny = pr.Ny, M = Nx - 2, L = Ny + 2;
-    double* W0 = a.work + a.woff[p];
-    batch_solve(W0, L, M, Ny / 2 + 1, pr.bc, pr.alpha, W0 + (int64_t)M * L);
+    const int2 g = a.groups[blockIdx.x];
+    const B2Prob pr = a.probs[g.x];
+    __shared__ double sm[kB2SolveLds];
+    batch_solve(a.work + a.woff[g.x], pr.Ny + 2, pr.Nx - 2, pr.Ny / 2 + 1, pr.bc, pr.alpha, g.y, 1 << 20, sm);
 }
 
 // ----------------------------------------------------------------- matrix builders
@@ -569,6 +695,7 @@ struct B2WideInfo {
     int cls[4];  // tile class of each stage
     int64_t ntask[4], off_task[4];
     int64_t off_probs, off_woff, work_doubles;
+    int64_t ngroup;  // column groups of the solve
     const double* mats;
 };
 static std::map<const void*, B2WideInfo> g_b2w;
@@ -743,8 +870,22 @@ static void b2_wide_order(int st, int cls, int nprob, const int* Nx, const int* 
 }
 
 // plan layout: problem table | tasks of each stage | per-problem workspace
-// offsets | solve order (problems by decreasing rows, the longest chains first)
-static int64_t b2_wide_bytes(int nprob, const int64_t ntask[4], int64_t off_task[4], int64_t* off_woff)
+// offsets | column groups of the solve
+static int leg_groups(int Nx, int Ny)
+{
+    const int tl = leg_solve_tl((Nx - 1) / 2);
+    return (Ny / 2 + tl) / tl;
+}
+
+static int64_t b2_wide_groups(int nprob, const int* Nx, const int* Ny)
+{
+    int64_t n = 0;
+    for (int i = 0; i < nprob; ++i) n += leg_groups(Nx[i], Ny[i]);
+    return n;
+}
+
+static int64_t b2_wide_bytes(int nprob, const int* Nx, const int* Ny, const int64_t ntask[4], int64_t off_task[4],
+                             int64_t* off_woff)
 {
     int64_t o = r256((int64_t)nprob * sizeof(B2Prob));
     for (int st = 0; st < 4; ++st) {
@@ -753,7 +894,7 @@ static int64_t b2_wide_bytes(int nprob, const int64_t ntask[4], int64_t off_task
     }
     *off_woff = o;
     o += r256((int64_t)nprob * 8);
-    return o + r256((int64_t)nprob * 4);  // the solve order after the offsets
+    return o + r256(b2_wide_groups(nprob, Nx, Ny) * (int64_t)sizeof(int2));
 }
 
 template <int BM, int BN, int BK>
@@ -932,7 +1073,7 @@ extern "C" int64_t sfa_batch2d_wide_plan_bytes(int nprob, const int* Nx, const i
     if (nprob < 1 || !Nx || !Ny) return -1;
     int64_t nt[4], ot[4], ow, work;
     b2_wide_shape(nprob, Nx, Ny, nt, &work);
-    return b2_wide_bytes(nprob, nt, ot, &ow);
+    return b2_wide_bytes(nprob, Nx, Ny, nt, ot, &ow);
 }
 
 extern "C" int64_t sfa_batch2d_wide_workspace(int nprob, const int* Nx, const int* Ny)
@@ -961,11 +1102,12 @@ extern "C" int sfa_batch2d_wide_plan(int nprob, const int* Nx, const int* Ny, co
     wi.nprob = nprob;
     int* cls = wi.cls;
     b2_wide_shape(nprob, Nx, Ny, wi.ntask, &wi.work_doubles, cls);
-    const int64_t bytes = b2_wide_bytes(nprob, wi.ntask, wi.off_task, &wi.off_woff);
+    const int64_t bytes = b2_wide_bytes(nprob, Nx, Ny, wi.ntask, wi.off_task, &wi.off_woff);
     SFA_CHECK(plan_bytes >= bytes, SFA_ERR_ARG, "plan buffer too small (%lld < %lld)",
               (long long)plan_bytes, (long long)bytes);
     wi.off_probs = 0;
     wi.mats = mats;
+    wi.ngroup = b2_wide_groups(nprob, Nx, Ny);
     std::vector<B2Task> tasks[4];
     for (int st = 0; st < 4; ++st) b2_wide_order(st, cls[st], nprob, Nx, Ny, wi.ntask[st], tasks[st]);
     std::vector<int64_t> woff(nprob);
@@ -982,12 +1124,16 @@ extern "C" int sfa_batch2d_wide_plan(int nprob, const int* Nx, const int* Ny, co
         SFA_HIP(hipMemcpyAsync(pb + wi.off_task[st], tasks[st].data(), tasks[st].size() * sizeof(B2Task),
                                hipMemcpyHostToDevice, s));
     SFA_HIP(hipMemcpyAsync(pb + wi.off_woff, woff.data(), woff.size() * 8, hipMemcpyHostToDevice, s));
-    // the solve's chains run sequentially over a problem's rows: the problems
-    // with the most rows start first so they do not finish last
+    // the solve takes the problems with the most rows first, so that they do not
+    // finish last
     std::vector<int> order(nprob);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return Nx[x] > Nx[y]; });
-    SFA_HIP(hipMemcpyAsync(pb + wi.off_woff + r256((int64_t)nprob * 8), order.data(), order.size() * 4,
+    std::vector<int2> groups;
+    groups.reserve((size_t)wi.ngroup);
+    for (int i : order)
+        for (int g = 0; g < leg_groups(Nx[i], Ny[i]); ++g) groups.push_back(make_int2(i, g));
+    SFA_HIP(hipMemcpyAsync(pb + wi.off_woff + r256((int64_t)nprob * 8), groups.data(), groups.size() * sizeof(int2),
                            hipMemcpyHostToDevice, s));
     SFA_HIP(hipStreamSynchronize(s));  // host vectors are copied before they go out of scope
     std::lock_guard<std::mutex> lk(g_b2_mu);
@@ -1015,7 +1161,7 @@ extern "C" int sfa_batch2d_wide_solve(const double* F, double* U, const void* pl
     a.U = U;
     a.probs = (const B2Prob*)pb;
     a.woff = (const int64_t*)(pb + wi.off_woff);
-    a.order = (const int*)(pb + wi.off_woff + r256((int64_t)wi.nprob * 8));
+    a.groups = (const int2*)(pb + wi.off_woff + r256((int64_t)wi.nprob * 8));
     a.mats = wi.mats;
     a.work = (double*)work;
     hipStream_t s = (hipStream_t)stream;
@@ -1025,7 +1171,7 @@ extern "C" int sfa_batch2d_wide_solve(const double* F, double* U, const void* pl
     if ((rc = launch_wide_stage<0>(a, wi.cls[0], wi.ntask[0], s))) return rc;
     a.tasks = (const B2Task*)(pb + wi.off_task[1]);
     if ((rc = launch_wide_stage<1>(a, wi.cls[1], wi.ntask[1], s))) return rc;
-    hipLaunchKernelGGL(batch2d_wide_solve_kernel, dim3((unsigned)wi.nprob), blk, 0, s, a);
+    hipLaunchKernelGGL(batch2d_wide_solve_kernel, dim3((unsigned)wi.ngroup), blk, 0, s, a);
     SFA_LAUNCH_CHECK();
     a.tasks = (const B2Task*)(pb + wi.off_task[2]);
     if ((rc = launch_wide_stage<2>(a, wi.cls[2], wi.ntask[2], s))) return rc;

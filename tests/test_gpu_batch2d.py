@@ -190,3 +190,39 @@ def test_batch2d_wide_large_tiles_and_autotune(sfa):
     print(f"  autotune: {tune['best']['label']} ({sorted(modes)})", flush=True)
     assert modes == {"persistent", "wide"}
     assert torch.equal(P(F), ref)
+
+
+@pytest.mark.parametrize("mode", ["wide", "persistent"])
+def test_batch2d_solve_segments(sfa, mode):
+    """The segmented per-ky solve at the edges of its row counts (2, 4, 6, 8 rows
+    per segment, 8, 4 or 2 columns per group, chains that end inside a segment,
+    at its end and one row into the next), with the Neumann gauge column and a
+    very large alpha, vs the oracle."""
+    nx = [8, 10, 66, 68, 130, 132, 194, 196, 258, 260, 386, 388, 514, 516, 1024]
+    ny = [4, 14, 16, 18, 30, 4, 14, 16, 18, 30, 4, 14, 16, 18, 4]
+    al = [0.0, 3.0, 0.0, 1e9, 0.5, 0.0, 40.0, 0.0, 1e9, 2.0, 0.0, 7.0, 0.0, 1.0, 0.0]
+    bc = ["N" if i % 2 == 0 else "D" for i in range(len(nx))]
+    rng = np.random.default_rng(11)
+    fs = [rng.standard_normal((a, b)) for a, b in zip(nx, ny)]
+    for f, a, b in zip(fs, al, bc):
+        if a == 0.0 and b == "N":
+            f -= f.mean(axis=1, keepdims=True)  # solvable: no mean along y
+    H = sfa.BatchedHelmholtz2D(nx, ny, al, bc, mode=mode)
+    def reference(f, a, b):
+        with np.errstate(all="ignore"):
+            u, fh, uh = S.legendre_fourier_2d(f, a, b)
+        if a == 0.0 and b == "N":
+            # the oracle has no gauge: column ky = 0 is diagonal (beta = 0), with u_0 = 0
+            n = f.shape[0]
+            k = np.arange(1, n - 2, dtype=float)
+            uh = uh.copy()
+            uh[0, 0] = 0.0
+            uh[1:n - 2, 0] = fh[1:n - 2, 0] / (2 * k * (k + 1) * (2 * k + 3) / ((k + 2) * (k + 3)))
+            uh[n - 2:] = 0.0
+            u = np.fft.irfft(S.basis_backward("legendre", "N", uh, 0), n=f.shape[1], axis=1) * f.shape[1]
+        return u
+
+    for n, a, b, f, u in zip(nx, al, bc, fs, H.unpack(H(H.pack(fs)))):
+        err = _rel(u, reference(f, a, b))
+        print(f"  {mode} Nx={n} alpha={a} bc={b}: max rel err {err:.2e}", flush=True)
+        assert err < 1e-11
