@@ -409,14 +409,17 @@ static const double* plan_lift(const void* plan)
     return it == g_plans.end() ? nullptr : it->second.lift;
 }
 
-// The x-pass on the plan's restart states for lengths with prime factors up to
-// 13; false where the length does not allow it.
+// The x-pass on the plan's restart states: one kernel for lengths with prime
+// factors up to 13, else a DCT-II, the solve and a DCT-III in place.  False above
+// 514 rows.
 static bool xpass_mix(double2* W, int Nx, int Ny, int Nzh, int Kp, double alpha, int neumann, const double* K2,
                       const XPlan& pv, int64_t nb, hipStream_t s, int* rc)
 {
     XMixArgs a;
     const int64_t E = segment_rows((Nx - 2 + 1) / 2);
-    if (E > 16 || nb > 65535 || !make_mix_plan(Nx, true, &a.plan)) return false;
+    if (E > 16 || nb > 65535) return false;
+    const bool one = make_mix_plan(Nx, true, &a.plan);
+    if (!one) a.plan = MixPlan{};
     a.W = W;
     a.sa = (int64_t)Ny * Kp;
     a.bstride = (int64_t)Nx * a.sa;
@@ -426,16 +429,22 @@ static bool xpass_mix(double2* W, int Nx, int Ny, int Nzh, int Kp, double alpha,
     a.Nzh = Nzh;
     a.N = Nx;
     const int nat = (Nx - 1) + (Nx - 1) / (2 * (int)E) + 1;  // natural order, padded
-    a.LS = (nat > a.plan.size() ? nat : a.plan.size()) | 1;  // odd: lines in distinct banks
+    a.LS = (one && a.plan.size() > nat ? a.plan.size() : nat) | 1;  // odd: lines in distinct banks
     if (xpass_mix_lds(a) > 160 * 1024) return false;
     a.neumann = neumann;
     a.alpha = alpha;
     a.K2 = K2;
     a.pl = pv;
-    a.tw = fft_table(Nx);
-    a.tq = quarter_table(Nx);
-    if (!a.tw || !a.tq) {
-        *rc = fail(SFA_ERR_HIP, "table allocation failed");
+    a.tw = a.tq = nullptr;
+    const int64_t shape[3] = {nb, Nx, a.sa}, str[3] = {a.bstride, a.sa, 1};
+    if (one) {
+        a.tw = fft_table(Nx);
+        a.tq = quarter_table(Nx);
+        if (!a.tw || !a.tq) {
+            *rc = fail(SFA_ERR_HIP, "table allocation failed");
+            return true;
+        }
+    } else if ((*rc = sfa_cheb_scalar_product(W, W, SFA_C128, 3, shape, str, str, 1, K2, (void*)s))) {
         return true;
     }
     switch (E) {
@@ -448,6 +457,7 @@ static bool xpass_mix(double2* W, int Nx, int Ny, int Nzh, int Kp, double alpha,
         case 12: *rc = xpass_mix_12(a, nb, s); break;
         default: *rc = xpass_mix_16(a, nb, s); break;
     }
+    if (!one && !*rc) *rc = sfa_cheb_backward(W, W, SFA_C128, 3, shape, str, str, 1, K2, (void*)s);
     return true;
 }
 

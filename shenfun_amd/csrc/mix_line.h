@@ -329,7 +329,8 @@ __global__ void __launch_bounds__(256) mix_kernel(MixArgs a)
 // 15.8 -> 8.9, 64 x 360 x 64 33.3 -> 13.7; R2C 180 x 150 x 200 42.2 -> 24.3,
 // 256 x 256 x 240 98.0 -> 51.7; DCT-II / DCT-III with stencil along axis 0
 // 192 x 96 x 81 34.2 / 38.1 -> 19.4 / 16.6, 256 x 256 x 129 162 / 186 -> 94 / 80.
-inline bool mix_setup(const LineArgs& la, MixArgs& a, unsigned* grid, unsigned* block, size_t* lds_bytes)
+inline bool mix_setup(const LineArgs& la, MixArgs& a, unsigned* grid, unsigned* block, size_t* lds_bytes,
+                      int most = 16)
 {
     const int nf = la.plan.nfft;
     int64_t d1 = la.d1, d2 = la.d2;
@@ -344,7 +345,7 @@ inline bool mix_setup(const LineArgs& la, MixArgs& a, unsigned* grid, unsigned* 
     if (!make_mix_plan(nf, !a.t_fast, &a.plan)) return false;
     const int64_t line = (int64_t)a.plan.size() * sizeof(double2);
     const int64_t table = (int64_t)nf * sizeof(double2);
-    int T = 16;
+    int T = most;  // lines at most
     while (T > 1 && T * line + table > 76 * 1024) T >>= 1;
     while (T > 1 && T >= 2 * d2) T >>= 1;
     while (T > 8 && d1 * ((d2 + T - 1) / T) < 512) T >>= 1;
@@ -401,13 +402,16 @@ int mix_run_dct3(bool cplx, const MixArgs& a, dim3 grid, dim3 block, size_t lds,
 int mix_run_dct1f(bool cplx, const MixArgs& a, dim3 grid, dim3 block, size_t lds, hipStream_t stream);
 int mix_run_dct1b(bool cplx, const MixArgs& a, dim3 grid, dim3 block, size_t lds, hipStream_t stream);
 
+// mix_blue.hip: lengths with larger prime factors, up to 2048
+bool blue_launch(int op, bool inv, const LineArgs& la, hipStream_t stream, int* rc);
+
 // Launch the mixed-radix form where the length allows it.
 inline bool mix_launch(int op, bool inv, const LineArgs& la, hipStream_t stream, int* rc)
 {
     MixArgs a;
     unsigned grid, block;
     size_t lds;
-    if (!mix_setup(la, a, &grid, &block, &lds)) return false;
+    if (!mix_setup(la, a, &grid, &block, &lds)) return blue_launch(op, inv, la, stream, rc);
     const bool c = la.in_cplx != 0;
     switch (op) {
         case OP_C2C: *rc = mix_run_fft(op, inv, a, grid, block, lds, stream); break;

@@ -150,15 +150,63 @@ __global__ void __launch_bounds__(XM_THREADS, E <= 6 ? 3 : 1) xpass_mix_kernel(X
     mix_rest<true>(pl, m, 0, a.tw, tid, nth, [](int, int) -> int64_t { return 0; }, 0, st);
 }
 
+// The solve alone, in place on the stencilled coefficients: for the lengths with
+// larger prime factors, between a DCT-II and a DCT-III of their own (three passes
+// over the array; 218 x 38 x 144 lines 1042 us in the form without a plan, 160
+// in this one).  The same workgroup and plan as above.
+template <int E>
+__global__ void __launch_bounds__(XM_THREADS) xsolve_kernel(XMixArgs a)
+{
+    extern __shared__ double2 smem[];
+    constexpr int T = XM_T, PADW = 2 * E;
+    auto pd = [](int k) { return k + k / PADW; };
+    const int tid = threadIdx.x;
+    const int N = a.N, M = N - 2, LS = a.LS;
+    const int64_t L0 = (int64_t)blockIdx.x * T, sa = a.sa;
+    double2* W = a.W + (int64_t)blockIdx.y * a.bstride + L0;
+    const int Tv = (int)((a.nl - L0) < T ? (a.nl - L0) : T);
+    const int t = tid >> 5, p = (tid >> 4) & 1, lane = tid & 15;
+    int u;
+    {
+        const uint32_t L = (uint32_t)(L0 + t), ky = L / (uint32_t)a.Kp, kz = L - ky * (uint32_t)a.Kp;
+        const bool ok = t < Tv && kz < (uint32_t)a.Nzh;
+        const int v = a.pl.linemap[ok ? ky * a.Nzh + kz : 0];
+        u = ok ? v : 0;
+    }
+    // lanes over lines for the array, over segments for the solve
+    const int tl = tid & (T - 1), r0 = tid >> 3, tc = tl < Tv ? tl : 0;
+#pragma unroll 4
+    for (int i = r0; i < M; i += XM_THREADS / T) lds_put(tl * LS + pd(i), W[tc + i * sa]);
+    const double be = a.alpha + a.pl.svals[u];
+    const double4 b4 = a.pl.bs[((int64_t)2 * u + p) * 16 + lane];
+    __syncthreads();
+    double2 f[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int i = 2 * (lane * E + e) + p;
+        const double2 v = lds_get(t * LS + pd(i < M ? i : 0));
+        f[e] = i < M ? v : make_double2(0.0, 0.0);
+    }
+    wave_sync();
+    helm_chain_solve_bs<E, 16, double2, PADW>(f, smem + t * LS, p, M, be, a.neumann != 0, b4, lane);
+    __syncthreads();
+    if (tl < Tv) {
+#pragma unroll 4
+        for (int i = r0; i < M; i += XM_THREADS / T) W[tl + i * sa] = lds_get(tl * LS + pd(i));
+        if (r0 < 2) W[tl + (M + r0) * sa] = make_double2(0.0, 0.0);  // boundary slots
+    }
+}
+
 inline size_t xpass_mix_lds(const XMixArgs& a)
 {
     return sizeof(double2) * ((size_t)XM_T * a.LS + 2 * (size_t)a.N + XM_T);
 }
 
+// The x-pass, or the solve alone where the plan has no passes (a.plan.np == 0).
 template <int E>
 int xpass_mix_run(const XMixArgs& a, int64_t nb, hipStream_t s)
 {
-    auto k = xpass_mix_kernel<E>;
+    auto k = a.plan.np ? xpass_mix_kernel<E> : xsolve_kernel<E>;
     const size_t lds = xpass_mix_lds(a);
     if (lds > 64 * 1024)
         SFA_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));

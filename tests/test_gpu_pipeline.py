@@ -85,10 +85,11 @@ def test_helmholtz3d_fused_repeat_identical(sfa):
 
 
 @pytest.mark.parametrize("bc,alpha", [("D", 0.0), ("N", 0.0), ("N", 2.0)])
-@pytest.mark.parametrize("Nx", [8, 9, 16, 33, 35, 66, 98, 99, 130, 132, 182, 195, 250, 260, 384, 390, 507])
+@pytest.mark.parametrize("Nx", [8, 9, 16, 17, 33, 35, 66, 67, 98, 99, 130, 132, 182, 195, 218, 250, 260, 384, 390, 507,
+                                509, 514])
 def test_helmholtz3d_xpass_lengths(sfa, Nx, bc, alpha):
     """The fused x-pass on every segment size (1, 2, 3, 4, 6, 8, 12, 16 rows,
-    lengths at both ends of each), odd lengths and a last workgroup of two
+    lengths at both ends of each), odd lengths, lengths with a large prime factor and a last workgroup of two
     lines, vs the oracle; alpha = 0 with Neumann ends is the gauge."""
     print(f"[xpass Nx={Nx} {bc} alpha={alpha}]", flush=True)
     f = S.helmholtz3d_rhs(Nx, 6, 4, seed=Nx)

@@ -362,3 +362,46 @@ def test_line_matmul_parity(sfa, parity, nout, nin, lines, cplx):
               _lib.arr(X.shape), _lib.arr(x.stride()), _lib.arr(y.stride()), 0, nout, _lib.ptr(m), parity,
               _lib.stream_ptr())
     assert rel(y, M @ X) < 1e-13
+
+
+@pytest.mark.parametrize("n", [17, 19, 31, 34, 109, 146, 218, 257, 313, 509, 998, 1021, 2039, 2048 + 34])
+@pytest.mark.parametrize("layout", [0, 1, 2])
+def test_large_prime_lines(sfa, n, layout):
+    """Lengths with a prime factor above 13 (Bluestein's algorithm up to 2048, one
+    length beyond it): C2C in place and out of place, R2C / C2R at n and 2 n,
+    both Chebyshev quadratures, real and complex, with and without a stencil."""
+    print(f"[large prime n={n} layout={layout}]", flush=True)
+    m = (5, 21) if n <= 400 else (1, 3)
+    def shp(k):
+        return ((k,) + m, (m[0], k, m[1]), m + (k,))[layout]
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(shp(n)) + 1j * rng.standard_normal(shp(n))
+    B = sfa.FunctionSpace(n, "F", dtype="D")
+    B.axis = layout
+    assert rel(B.scalar_product(dev(x)), np.fft.fft(x, axis=layout) / n) < TOL
+    y = dev(x)
+    B.backward(y, y)
+    assert rel(y, np.fft.ifft(x, axis=layout) * n) < TOL
+    for k in (n, 2 * n):
+        r = rng.standard_normal(shp(k))
+        R = sfa.FunctionSpace(k, "F", dtype="d")
+        R.axis = layout
+        c = np.fft.rfft(r, axis=layout)
+        assert rel(R.scalar_product(dev(r)), c / k) < TOL
+        assert rel(R.backward(dev(c)), r * k) < TOL
+    for bc in (None, "D", "N"):
+        for quad, N in (("GC", n), ("GL", n // 2 + 1)):  # GL: FFT length 2 (N - 1)
+            z0 = rng.standard_normal(shp(N)) + 1j * rng.standard_normal(shp(N))
+            for z in (z0, z0.real.copy()):
+                V = sfa.FunctionSpace(N, "chebyshev", bc=bc, quad=quad)
+                V.axis = layout
+                ref = S.basis_scalar_product("chebyshev", bc, z, layout, quad=quad)
+                y = dev(z)
+                assert rel(V.scalar_product(y, kind="fast"), ref) < TOL
+                V.scalar_product(y, y, kind="fast")
+                assert rel(y, ref) < TOL
+                if bc is not None:
+                    z = z.copy()
+                    np.moveaxis(z, layout, 0)[N - 2:] = 0
+                assert rel(V.backward(dev(z), kind="fast"),
+                           S.basis_backward("chebyshev", bc, z, layout, quad=quad)) < TOL
