@@ -226,6 +226,13 @@ int sfa_pdma_lu(double* data, int64_t n, int64_t nbatch, void* stream);
 int sfa_tdma_solve(void* u, int dtype, int ndim, const int64_t* shape,
                    const int64_t* strides, int axis, const double* data, int64_t n,
                    int64_t data_line_stride, int64_t skip_lines, void* stream);
+
+/* sfa_tdma_solve with one set of factors, the nzero rows after the n of the
+ * system set to zero (the boundary slots of a forward transform:
+ * tensorproductspace.py:2091-2106 and the inverse mass matrix,
+ * spectralbase.py:560-577, in one pass). */
+int sfa_tdma_mass_solve(void* u, int dtype, int ndim, const int64_t* shape, const int64_t* strides,
+                        int axis, const double* data, int64_t n, int64_t nzero, void* stream);
 int sfa_pdma_solve(void* u, int dtype, int ndim, const int64_t* shape,
                    const int64_t* strides, int axis, const double* data, int64_t n,
                    int64_t data_line_stride, int64_t skip_lines, void* stream);

@@ -36,6 +36,7 @@ _SIGS = {
     "sfa_tdma_lu": "vllv",
     "sfa_pdma_lu": "vllv",
     "sfa_tdma_solve": "viiaaivlllv",
+    "sfa_tdma_mass_solve": "viiaaivllv",
     "sfa_pdma_solve": "viiaaivlllv",
     "sfa_diagma_solve": "viiaaivlllv",
     "sfa_pad_axis": "vviiaaaaiiillllv",

@@ -607,6 +607,14 @@ class _PolyBase(SpectralBase):
         tensorproductspace.py:2091-2106)."""
         out = self.scalar_product(input_array, output_array, kind)
         if self.is_composite:
+            solver = self._mass_solver()
+            if not self.has_nonhomogeneous_bcs and solver.solve_fn == "sfa_tdma_solve":
+                # zero boundary slots and the solve in one launch
+                lu = solver.perform_lu(out.device)
+                shp, st = _geom(out)
+                _lib.call("sfa_tdma_mass_solve", _lib.ptr(out), self._dtype_code(out), out.dim(), shp, st,
+                          self.axis, _lib.ptr(lu), self.dim(), self.N - self.dim(), _lib.stream_ptr())
+                return out
             self.set_boundary_dofs(out)
             if self.has_nonhomogeneous_bcs:
                 # _add_mass_rhs (tensorproductspace.py:2091-2106): minus the

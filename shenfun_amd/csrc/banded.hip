@@ -496,6 +496,7 @@ struct ChainArgs {
     T* u;
     LineMap gb, gu;
     int n;            // rows of the system
+    int zero;         // rows after them set to zero (boundary slots)
     int64_t skip;     // lines below it are left alone
     // TDMA: DIA rows of la.pyx:243-252's LU, line L at data + L dls
     const double* data;
@@ -547,6 +548,9 @@ __global__ void __launch_bounds__(256) chain_solve_kernel(ChainArgs<T> g)
     }
     const int K = (n - p + 1) / 2;  // rows i = p + 2 m, m < K
     const int nch = ONE ? 1 : (K + SG * E - 1) / (SG * E);
+
+    if (valid && seg == 0)
+        for (int i = n + p; i < n + g.zero; i += 2) ul[(int64_t)i * su] = zero<T>();
 
     T y[E];
     double iv[E], q[E], w[HELM ? E : 1];
@@ -801,9 +805,10 @@ using namespace sfa;
 
 template <typename T>
 static ChainArgs<T> tdma_args(T* u, const LineMap& g, const double* data, int64_t n, int64_t dls,
-                              int64_t skip)
+                              int64_t skip, int nzero)
 {
     ChainArgs<T> a{};
+    a.zero = nzero;
     a.b = u;
     a.u = u;
     a.gb = a.gu = g;
@@ -817,7 +822,7 @@ static ChainArgs<T> tdma_args(T* u, const LineMap& g, const double* data, int64_
 template <int KIND>
 static int banded_solve(void* u, int dtype, int ndim, const int64_t* shape, const int64_t* strides,
                         int axis, const double* data, int64_t n, int64_t dls, int64_t skip,
-                        void* stream)
+                        void* stream, int64_t nzero = 0)
 {
     LineMap g;
     int64_t len;
@@ -829,6 +834,8 @@ static int banded_solve(void* u, int dtype, int ndim, const int64_t* shape, cons
     SFA_CHECK(KIND == 0 || n >= (KIND == 1 ? 2 : 4), SFA_ERR_ARG, "system too small (n=%lld)",
               (long long)n);
     SFA_CHECK(dls >= 0 && skip >= 0, SFA_ERR_ARG, "negative stride/skip");
+    SFA_CHECK(nzero >= 0 && n + nzero <= len, SFA_ERR_ARG, "%lld rows and %lld zeroed ones on a line of %lld",
+              (long long)n, (long long)nzero, (long long)len);
     const int bs = 256;
     auto absl = [](int64_t v) { return v < 0 ? -v : v; };
     const int along = absl(g.sa) <= absl(g.s2) ? 1 : 0;
@@ -839,12 +846,12 @@ static int banded_solve(void* u, int dtype, int ndim, const int64_t* shape, cons
     if (dtype == SFA_C128) {
         double2* uu = (double2*)u;
         if (KIND == 0) hipLaunchKernelGGL(diag_solve_kernel<double2>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip, along);
-        if (KIND == 1) chain_launch<double2, false>(tdma_args(uu, g, data, n, dls, skip), s);
+        if (KIND == 1) chain_launch<double2, false>(tdma_args(uu, g, data, n, dls, skip, (int)nzero), s);
         if (KIND == 2) hipLaunchKernelGGL(pdma_solve_kernel<double2>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip);
     } else {
         double* uu = (double*)u;
         if (KIND == 0) hipLaunchKernelGGL(diag_solve_kernel<double>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip, along);
-        if (KIND == 1) chain_launch<double, false>(tdma_args(uu, g, data, n, dls, skip), s);
+        if (KIND == 1) chain_launch<double, false>(tdma_args(uu, g, data, n, dls, skip, (int)nzero), s);
         if (KIND == 2) hipLaunchKernelGGL(pdma_solve_kernel<double>, grid, dim3(bs), 0, s, uu, g, data, (int)n, dls, skip);
     }
     SFA_LAUNCH_CHECK();
@@ -857,6 +864,12 @@ extern "C" int sfa_tdma_solve(void* u, int dtype, int ndim, const int64_t* shape
 {
     return banded_solve<1>(u, dtype, ndim, shape, strides, axis, data, n, data_line_stride,
                            skip_lines, stream);
+}
+
+extern "C" int sfa_tdma_mass_solve(void* u, int dtype, int ndim, const int64_t* shape, const int64_t* strides,
+                                   int axis, const double* data, int64_t n, int64_t nzero, void* stream)
+{
+    return banded_solve<1>(u, dtype, ndim, shape, strides, axis, data, n, 0, 0, stream, nzero);
 }
 
 extern "C" int sfa_pdma_solve(void* u, int dtype, int ndim, const int64_t* shape,

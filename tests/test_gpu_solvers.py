@@ -328,3 +328,25 @@ def test_chain_scan_zero_lines(sfa):
     b = np.zeros((n, 3))
     u = sfa.la.TDMA(sfa.SparseMatrix(d3, (n, n)))(dev(b), axis=0)
     assert torch.equal(u, torch.zeros_like(u))
+
+
+@pytest.mark.parametrize("shape,axis", [((12,), 0), ((9, 40, 60), 0), ((5, 33, 7), 1), ((3, 700), 1)])
+def test_tdma_mass_solve(sfa, shape, axis):
+    """sfa_tdma_mass_solve: the solve's bits, the rows after the system zero, a
+    system that would not fit its line refused."""
+    from shenfun_amd import _lib
+    rng = np.random.default_rng(shape[axis])
+    N = shape[axis]
+    n = N - 2
+    d3 = {0: rng.uniform(2, 3, n), -2: rng.uniform(0.1, 1, n - 2), 2: rng.uniform(0.1, 1, n - 2)}
+    lu = dev(S.tdma_lu(S.tdma_dia(d3, n)))
+    b = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    u, v = dev(b), dev(b)
+    args = lambda t: (_lib.ptr(t), _lib.C128, t.dim(), _lib.arr(t.shape), _lib.arr(t.stride()), axis,  # noqa: E731
+                      _lib.ptr(lu))
+    _lib.call("sfa_tdma_solve", *args(u), n, 0, 0, _lib.stream_ptr())
+    _lib.call("sfa_tdma_mass_solve", *args(v), n, 2, _lib.stream_ptr())
+    assert torch.equal(v.narrow(axis, 0, n), u.narrow(axis, 0, n))
+    assert not bool(v.narrow(axis, n, 2).any())
+    with pytest.raises(RuntimeError):
+        _lib.call("sfa_tdma_mass_solve", *args(v), n, 3, _lib.stream_ptr())
