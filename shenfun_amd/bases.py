@@ -13,6 +13,8 @@ Mirrors the per-axis SpectralBase interface (spectralbase.py:200-313):
 
 Compute runs only through the C ABI of libshenfun_amd.so.
 """
+import math
+
 import numpy as np
 import torch
 
@@ -165,7 +167,7 @@ class SpectralBase(_Planned):
 
     def _phys_len(self):
         if self.padding_factor != 1:
-            return int(np.floor(self.padding_factor * self.N))
+            return math.floor(self.padding_factor * self.N)
         return self.N
 
     def get_dealiased(self, padding_factor=1.5, dealias_direct=False, **kw):
