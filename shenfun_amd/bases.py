@@ -350,6 +350,32 @@ class _PolyBase(SpectralBase):
     def _synthesis_matrix(self):
         raise NotImplementedError
 
+    def _dense(self, kind, inp, out):
+        """Whether the transform of this kind is a dense contraction."""
+        return True
+
+    @staticmethod
+    def _padded_dense(twin, kind, inp, out):
+        # (arrays of one storage may overlap: those go through a temporary)
+        return twin._dense(kind, inp, out) and \
+            inp.untyped_storage().data_ptr() != out.untyped_storage().data_ptr()
+
+    def _padded_matrix(self, which, twin):
+        """The padded-length twin's analysis rows ('a') or synthesis columns
+        ('s') of this space's own functions, zero for the boundary slots: the
+        padding or truncation of the coefficients inside the product."""
+        key = ("padded", which)
+        if key not in self._cache:
+            n = self.dim()
+            if which == "a":
+                M = torch.zeros((self.N, twin.N), dtype=torch.float64, device=self.device)
+                M[:n] = twin._analysis_matrix()[:n]
+            else:
+                M = torch.zeros((twin.N, self.N), dtype=torch.float64, device=self.device)
+                M[:, :n] = twin._synthesis_matrix()[:, :n]
+            self._cache[key] = M
+        return self._cache[key]
+
     # ------------------------------------------------------------ transforms
     def _clone(self, N, padding_factor=1, dealias_direct=False):
         return type(self)(N, quad=self.quad, bc=self._bc_orig, dtype=self.dtype,
@@ -561,8 +587,12 @@ class _PolyBase(SpectralBase):
         if self.is_padded:
             # padded-length scalar product, truncated to the N coefficients
             # (spectralbase.py:225-229, _truncation_forward :1362-1366)
+            twin = self._twin()
+            if self._padded_dense(twin, kind, inp, out):  # the kept rows of its matrix, in one product
+                self._matmul(inp, out, self._padded_matrix("a", twin), 1)
+                return out
             tmp = self._tmp("sp", inp.shape, inp.dtype)
-            self._twin()._scalar_product(inp, tmp, kind)
+            twin._scalar_product(inp, tmp, kind)
             self._pad(tmp, out, 1, self.N - self.dim())
             return out
         self._scalar_product(inp, out, kind)
@@ -583,10 +613,14 @@ class _PolyBase(SpectralBase):
             # zero-padded coefficients, boundary slots moved to the end
             # (_padding_backward, spectralbase.py:1368-1389), then the
             # padded-length synthesis
-            shp = list(inp.shape)
-            shp[self.axis] = self._phys_len()
-            tmp = self._pad(inp, self._tmp("bw", shp, inp.dtype), 0, nbc)
-            self._twin()._backward(tmp, out, kind)
+            twin = self._twin()
+            if self._padded_dense(twin, kind, inp, out):
+                self._matmul(inp, out, self._padded_matrix("s", twin), 2)
+            else:
+                shp = list(inp.shape)
+                shp[self.axis] = self._phys_len()
+                tmp = self._pad(inp, self._tmp("bw", shp, inp.dtype), 0, nbc)
+                twin._backward(tmp, out, kind)
         else:
             if self.dealias_direct:
                 inp = self._dealias_input(inp, nbc)
@@ -667,9 +701,18 @@ class ChebyshevBase(_PolyBase):
         return h
 
     def _vander(self):
-        x, _ = self.points_and_weights(self.N)
-        j = np.arange(self.N)
-        return np.cos(np.outer(np.arccos(x), j))  # T_k(x_j) = cos(k theta_j)
+        """T_k(x_j) = cos(k theta_j), the angles reduced in integers so that
+        every entry is as exact, and the matrix as even and odd, as cos is."""
+        j, k = np.arange(self.N)[:, None], np.arange(self.N)[None, :]
+        if self.quad == "GL":  # theta_j = pi j / (N - 1)
+            m, q = j * k, self.N - 1
+        else:  # pi (2j + 1) / (2N)
+            m, q = (2 * j + 1) * k, 2 * self.N
+        m = m % (2 * q)
+        m = np.minimum(m, 2 * q - m)  # cos(2 pi - t) = cos t
+        sign = np.where(2 * m > q, -1.0, 1.0)
+        m = np.where(2 * m > q, q - m, m)  # cos(pi - t) = -cos t
+        return np.where(2 * m == q, 0.0, sign * np.cos(PI * m / q))
 
     def _analysis_matrix(self):
         def build():
@@ -705,6 +748,9 @@ class ChebyshevBase(_PolyBase):
             return kind
         dense = self._phys_len() <= self.DENSE_MAX and out.data_ptr() != inp.data_ptr()
         return "vandermonde" if dense else "fast"
+
+    def _dense(self, kind, inp, out):
+        return self._auto(kind, inp, out) not in ("fast", "hip")
 
     def _scalar_product(self, inp, out, kind):
         kind = self._auto(kind, inp, out)
@@ -1203,6 +1249,9 @@ class _StencilSpace:
     def _ortho_vander(self):
         x, w = self.points_and_weights(self.N)
         return self._vander_at(x, self.N), w
+
+    def _dense(self, kind, inp, out):
+        return True
 
     def _analysis_matrix(self):
         def build():
