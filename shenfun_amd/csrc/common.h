@@ -104,6 +104,8 @@ int make_geom(int ndim, const int64_t* shape, const int64_t* strides, int axis, 
 // fft_table(n): w[m] = exp(-2 pi i m / n), m = 0..n-1.
 // quarter_table(N): w[k] = exp(-i pi k / (2N)), k = 0..N-1.
 const double2* fft_table(int n);
+// every table that complex lines of length nf read (mix_blue.hip)
+int line_tables(int nf);
 const double2* quarter_table(int N);
 
 // While a NoAllocScope lives on this host thread, the lazily built device

@@ -356,6 +356,21 @@ static bool blue_table(int nf, BlueTable* out, int* rc)
     return true;
 }
 
+// Tables of the complex lines of length nf that no plan of the caller holds:
+// a pipeline that is captured into a graph right after its plan was made may
+// not allocate them then.
+int line_tables(int nf)
+{
+    SFA_CHECK(fft_table(nf) != nullptr, SFA_ERR_HIP, "table allocation failed");
+    MixPlan p;
+    if (make_mix_plan(nf, true, &p) || nf > 2048) return SFA_OK;
+    int rc = SFA_OK;
+    BlueTable tab{0, nullptr};
+    if (!blue_table(nf, &tab, &rc)) return SFA_OK;
+    SFA_CHECK(rc || fft_table(tab.M) != nullptr, SFA_ERR_HIP, "table allocation failed");
+    return rc;
+}
+
 bool blue_launch(int op, bool inv, const LineArgs& la, hipStream_t stream, int* rc)
 {
     BlueArgs ba;

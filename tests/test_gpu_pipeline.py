@@ -100,6 +100,32 @@ def test_helmholtz3d_xpass_lengths(sfa, Nx, bc, alpha):
     assert rel(u, S.helmholtz3d_cheb_fourier(f, alpha, bc)[0]) < 1e-12
 
 
+@pytest.mark.parametrize("shape", [(62, 74, 86), (93, 111, 134)])
+def test_helmholtz3d_first_solve_captured(sfa, shape):
+    """The first solve of lengths with a prime factor above 13 (their chirp
+    tables are of no other test) is captured in a HIP graph right after the
+    plan was made: every replay equals the eager result."""
+    print(f"[first solve captured {shape}]", flush=True)
+    f = S.helmholtz3d_rhs(*shape, seed=3)
+    T = sfa.TensorProductSpace(None, (sfa.FunctionSpace(shape[0], "chebyshev", bc="D"),
+                                      sfa.FunctionSpace(shape[1], "F", dtype="D"),
+                                      sfa.FunctionSpace(shape[2], "F", dtype="d")))
+    H = sfa.HelmholtzSolver3D(T, 2.0)
+    fd = dev(f)
+    u = torch.empty_like(fd)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        H(fd, u)
+    for _ in range(3):
+        u.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel(u, S.helmholtz3d_cheb_fourier(f, 2.0, "D")[0]) < 1e-12
+        eager = H(fd)
+        assert torch.equal(eager, u)
+
+
 @pytest.mark.parametrize("precision,shape,bc", [("fp64", (32, 24, 16), "D"), ("fp64", (64, 20, 16), "N"),
                                                ("fp64", (64, 16, 128), "D"), ("mixed", (64, 32, 64), "D"),
                                                ("mixed", (128, 16, 64), "N")])
