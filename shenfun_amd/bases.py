@@ -373,6 +373,7 @@ class _PolyBase(SpectralBase):
             else:
                 M = torch.zeros((twin.N, self.N), dtype=torch.float64, device=self.device)
                 M[:, :n] = twin._synthesis_matrix()[:, :n]
+            torch.cuda.current_stream(M.device).synchronize()  # other streams may take it from the cache
             self._cache[key] = M
         return self._cache[key]
 
@@ -708,11 +709,12 @@ class ChebyshevBase(_PolyBase):
             m, q = j * k, self.N - 1
         else:  # pi (2j + 1) / (2N)
             m, q = (2 * j + 1) * k, 2 * self.N
-        m = m % (2 * q)
-        m = np.minimum(m, 2 * q - m)  # cos(2 pi - t) = cos t
-        sign = np.where(2 * m > q, -1.0, 1.0)
-        m = np.where(2 * m > q, q - m, m)  # cos(pi - t) = -cos t
-        return np.where(2 * m == q, 0.0, sign * np.cos(PI * m / q))
+        t = np.arange(2 * q)
+        t = np.minimum(t, 2 * q - t)  # cos(2 pi - a) = cos a
+        sign = np.where(2 * t > q, -1.0, 1.0)
+        t = np.where(2 * t > q, q - t, t)  # cos(pi - a) = -cos a
+        c = np.where(2 * t == q, 0.0, sign * np.cos(PI * t / q))
+        return np.take(c, m - m // (2 * q) * (2 * q))
 
     def _analysis_matrix(self):
         def build():
@@ -737,10 +739,10 @@ class ChebyshevBase(_PolyBase):
         return self._dev_array("Ms", build)
 
     # 'auto': up to this many points the transforms run as dense contractions
-    # on FP64 MFMA (sfa_line_matmul); above it as DCTs on the complex FFT
-    # kernels.  Measured on the MI355X along axis 0 of (N, N, N/2 + 1) arrays:
-    # N = 128 scalar product 21.7 us dense vs 26.0 us DCT, backward 21.7 vs
-    # 32.5; N = 256 scalar product 197 vs 164 (the DCT wins).
+    # on FP64 MFMA (sfa_line_matmul_parity); above it as DCTs on the complex FFT
+    # kernels.  Measured on the MI355X along axis 0 of (N, N, N/2 + 1) arrays,
+    # scalar product / backward: N = 64 dense 8.2 / 8.6 us, DCT 10.5 / 8.8;
+    # N = 128 15.7 / 14.9 and 16.6 / 14.5; N = 256 132 / 115 and 98 / 84.
     DENSE_MAX = 128
 
     def _auto(self, kind, inp, out):
