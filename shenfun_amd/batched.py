@@ -265,12 +265,15 @@ class BatchedHelmholtz2D:
 
     def flops(self):
         """FP64 flops the kernel executes per batch: the four contractions
-        (two Legendre, two dense real DFT), 2 per multiply-add."""
+        (two Legendre, two dense real DFT), 2 per multiply-add, each over half
+        of its inner length (the sums and differences of mirrored values)."""
         nx = self.Nx.astype(float)
         ny = self.Ny.astype(float)
+        hx = (nx + 1) // 2
+        hy = ny // 2 + 1
         m = nx - 2
         L = ny + 2
-        return float(np.sum(2 * m * nx * ny + 2 * m * ny * L + 2 * nx * m * L + 2 * nx * L * ny))
+        return float(np.sum(2 * m * hx * ny + 2 * m * hy * L + 2 * hx * m * L + 2 * nx * L * hy))
 
     def bytes_moved(self):
         """Compulsory HBM bytes per batch: f read and u written once."""

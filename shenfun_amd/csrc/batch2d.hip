@@ -15,7 +15,10 @@
 //   u = U1 Di               C2R along y (imag of k = 0 and Nyquist ignored)
 // Phi[j, m] = L_m(x_j) + K2_m L_{m+2}(x_j) on the Legendre-Gauss nodes; Df, Di
 // are the real DFT matrices.  All four contractions are FP64 GEMMs on MFMA
-// (v_mfma_f64_16x16x4f64).  One workgroup owns a problem from start to end; the
+// (v_mfma_f64_16x16x4f64), each over half of its inner length: the points are
+// symmetric, so even and odd functions act on the sums and differences of
+// mirrored values (fold_tile).  The per-ky solves are segmented scans
+// (leg_solve_group).  One workgroup owns a problem from start to end; the
 // host assigns problems to workgroups largest first (static LPT schedule), so
 // the launch needs no atomics and every workgroup exits after its list.
 #include <algorithm>

@@ -9,8 +9,8 @@ device memory free up, so work of several requests overlaps on the device:
   (one line per request), then one scalar-product, one Helmholtz-solve and one
   backward launch.  A batch whose requests share one alpha that has been seen
   before uses the cached factors of (N, bc, alpha) instead, broadcast to every
-  line; an alpha seen once fills no cache entry.  Lengths with a prime factor above 31 (whose mixed-radix
-  DCT degenerates to an O(N p) DFT) use the cached dense transform matrices
+  line; an alpha seen once fills no cache entry.  Lengths with a prime factor above 31 (Bluestein
+  lines up to 2048 points, an O(N p) DFT past that) use the cached dense transform matrices
   instead (the matrix kind of spectralbase.py:484-491, 550-558).  Reference
   path per request: chebyshev.bases scalar_product
   (chebyshev/bases.py:340-353) -> chebyshev.la.Helmholtz (chebyshev/la.py:
