@@ -34,6 +34,17 @@ struct LineMap {
     }
 };
 
+// A launch may have at most 2^32 - 1 work items along x: grids of more than
+// kWideX workgroups of 256 go on along z (wide_grid; the last of them may be
+// past the end), and a kernel asks for its workgroup's number with wide_block.
+constexpr int64_t kWideX = 1 << 23;
+__device__ inline int64_t wide_block() { return (int64_t)blockIdx.z * gridDim.x + blockIdx.x; }
+static inline dim3 wide_grid(int64_t nblk, unsigned y)
+{
+    const int64_t z = (nblk + kWideX - 1) / kWideX;
+    return dim3((unsigned)((nblk + z - 1) / z), y, (unsigned)z);
+}
+
 __device__ inline int last_of_parity(int n, int p) { return (n - 1) - (((n - 1) - p) & 1); }
 
 // ----------------------------------------------------------------- TDMA
@@ -141,7 +152,7 @@ template <typename T>
 __global__ void diag_solve_kernel(T* __restrict__ u, LineMap g, const double* __restrict__ dd,
                                   int n, int64_t dls, int64_t skip, int along)
 {
-    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t gid = wide_block() * blockDim.x + threadIdx.x;
     if (gid >= g.nlines * n) return;
     const int64_t L = along ? gid / n : gid % g.nlines;
     const int i = (int)(along ? gid - L * n : gid / g.nlines);
@@ -524,7 +535,7 @@ __global__ void __launch_bounds__(256) chain_solve_kernel(ChainArgs<T> g)
     __shared__ T sC[NW][TL][2];
     const int tid = threadIdx.x, t = tid % TL, seg = tid / TL, wave = tid >> 6, ws = seg % WS;
     const int p = blockIdx.y, n = g.n;
-    const int64_t L = (int64_t)blockIdx.x * TL + t;
+    const int64_t L = wide_block() * TL + t;
     const bool valid = L < g.gu.nlines && L >= g.skip;
     const int64_t Lc = valid ? L : 0;
     const T* bl = g.b + g.gb.off(Lc);
@@ -754,7 +765,7 @@ static void chain_launch_tl(const ChainArgs<T>& a, hipStream_t s)
 {
     constexpr int SG = 256 / TL;
     const int K = (a.n + 1) / 2;
-    const dim3 grid((unsigned)((a.gu.nlines + TL - 1) / TL), 2), block(256);
+    const dim3 grid = wide_grid((a.gu.nlines + TL - 1) / TL, 2), block(256);
     if (K <= SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 1, HELM, true>), grid, block, 0, s, a);
     else if (K <= 2 * SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 2, HELM, true>), grid, block, 0, s, a);
     else if (K <= 4 * SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 4, HELM, true>), grid, block, 0, s, a);
@@ -839,9 +850,11 @@ static int banded_solve(void* u, int dtype, int ndim, const int64_t* shape, cons
     const int bs = 256;
     auto absl = [](int64_t v) { return v < 0 ? -v : v; };
     const int along = absl(g.sa) <= absl(g.s2) ? 1 : 0;
-    const int64_t nth = KIND == 0 ? g.nlines * n : 2 * g.nlines;
-    SFA_CHECK((nth + bs - 1) / bs < (1ll << 31), SFA_ERR_UNSUPPORTED, "too many lines");
-    dim3 grid = grid_for(nth, bs);
+    dim3 grid = wide_grid((g.nlines * n + bs - 1) / bs, 1);  // DiagMA
+    if (KIND == 2) {
+        SFA_CHECK(2 * g.nlines < (1ll << 32), SFA_ERR_UNSUPPORTED, "too many lines");
+        grid = grid_for(2 * g.nlines, bs);
+    }
     hipStream_t s = (hipStream_t)stream;
     if (dtype == SFA_C128) {
         double2* uu = (double2*)u;

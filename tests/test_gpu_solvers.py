@@ -350,3 +350,37 @@ def test_tdma_mass_solve(sfa, shape, axis):
     assert not bool(v.narrow(axis, n, 2).any())
     with pytest.raises(RuntimeError):
         _lib.call("sfa_tdma_mass_solve", *args(v), n, 3, _lib.stream_ptr())
+
+
+@pytest.mark.parametrize("kind", ["TDMA", "Helmholtz", "DiagMA"])
+def test_solve_line_counts_past_one_grid(sfa, kind):
+    """Many short contiguous lines: more workgroups (or, for the elementwise
+    solve, threads) than one dimension of a launch may hold.  The lines repeat
+    64 different ones, so every block of 64 has their solution."""
+    print(f"[line counts past one grid: {kind}]", flush=True)
+    from shenfun_amd import _lib
+    N, reps = 8, (1 << 23 if kind == "DiagMA" else 1 << 21) + 1
+    if torch.cuda.mem_get_info()[0] < 3 * 64 * reps * N * 8:
+        pytest.skip("needs three arrays of the size")
+    rng = np.random.default_rng(5)
+    b = rng.standard_normal((64, N))
+    u = dev(b).repeat(reps, 1)
+    if kind == "Helmholtz":
+        f = S.helmholtz_lu("D", N, -np.ones(1), np.full(1, 3.0))
+        ref = S.helmholtz_solve(b.T.copy(), *f, neumann=False).T
+        fd = [dev(np.ascontiguousarray(x.reshape(-1))) for x in f]
+        _lib.call("sfa_helmholtz_solve", _lib.ptr(u), _lib.ptr(u), _lib.F64, 2, _lib.arr(u.shape),
+                  _lib.arr(u.stride()), _lib.arr(u.stride()), 1, 0, *[_lib.ptr(x) for x in fd],
+                  _lib.arr((0, 1)), _lib.stream_ptr())
+    else:
+        d = {0: rng.uniform(2, 3, N)}
+        if kind == "TDMA":
+            d.update({-2: rng.uniform(0.1, 1, N - 2), 2: rng.uniform(0.1, 1, N - 2)})
+            ref = S.tdma_solve(b, S.tdma_lu(S.tdma_dia(d, N)), 1)
+        else:
+            ref = b / d[0]
+        getattr(sfa.la, kind)(sfa.SparseMatrix(d, (N, N)))(u, axis=1)
+    n = N - 2 if kind == "Helmholtz" else N
+    u = u.view(reps, 64, N)[:, :, :n]
+    r = dev(np.ascontiguousarray(ref[:, :n]))
+    assert float((u - r).abs_().amax()) < TOL * float(r.abs().max())
