@@ -34,17 +34,6 @@ struct LineMap {
     }
 };
 
-// A launch may have at most 2^32 - 1 work items along x: grids of more than
-// kWideX workgroups of 256 go on along z (wide_grid; the last of them may be
-// past the end), and a kernel asks for its workgroup's number with wide_block.
-constexpr int64_t kWideX = 1 << 23;
-__device__ inline int64_t wide_block() { return (int64_t)blockIdx.z * gridDim.x + blockIdx.x; }
-static inline dim3 wide_grid(int64_t nblk, unsigned y)
-{
-    const int64_t z = (nblk + kWideX - 1) / kWideX;
-    return dim3((unsigned)((nblk + z - 1) / z), y, (unsigned)z);
-}
-
 __device__ inline int last_of_parity(int n, int p) { return (n - 1) - (((n - 1) - p) & 1); }
 
 // ----------------------------------------------------------------- TDMA

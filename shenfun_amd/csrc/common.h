@@ -100,6 +100,18 @@ struct Geom {
 // Build a Geom from (ndim, shape, strides, axis).  Returns 0 or an error.
 int make_geom(int ndim, const int64_t* shape, const int64_t* strides, int axis, Geom* g);
 
+// A launch of 2^32 or more work items along x runs only part of them, without an
+// error: grids of more than kWideX workgroups (of at most 256 threads) go on
+// along z.  A kernel asks for its workgroup's number with wide_block; the last
+// ones may be past the end.
+constexpr int64_t kWideX = 1 << 23;
+__device__ inline int64_t wide_block() { return (int64_t)blockIdx.z * gridDim.x + blockIdx.x; }
+static inline dim3 wide_grid(int64_t nblk, unsigned y = 1)
+{
+    const int64_t z = (nblk + kWideX - 1) / kWideX;
+    return dim3((unsigned)((nblk + z - 1) / z), y, (unsigned)z);
+}
+
 // Device twiddle tables, cached per length for the process lifetime.
 // fft_table(n): w[m] = exp(-2 pi i m / n), m = 0..n-1.
 // quarter_table(N): w[k] = exp(-i pi k / (2N)), k = 0..N-1.

@@ -39,8 +39,9 @@ __global__ void __launch_bounds__(256) blue_kernel(BlueArgs ba)
     const MixArgs& a = ba.a;
     const int tid = threadIdx.x, nth = blockDim.x;
     const int64_t ntile = (a.d2 + a.T - 1) / a.T;
-    const int64_t i1 = blockIdx.x / ntile;
-    const int64_t t0 = (blockIdx.x - i1 * ntile) * a.T;
+    const int64_t blk = wide_block(), i1 = blk / ntile;
+    if (i1 >= a.d1) return;
+    const int64_t t0 = (blk - i1 * ntile) * a.T;
     const MixPlan& pl = a.plan;
     MixTile m;
     m.T = a.T;
@@ -383,7 +384,8 @@ bool blue_launch(int op, bool inv, const LineArgs& la, hipStream_t stream, int* 
     if (*rc) return true;
     LineArgs lb = la;
     lb.plan.nfft = tab.M;
-    unsigned grid, block;
+    dim3 grid;
+    unsigned block;
     size_t lds;
     int most = 16;
     while (most > 1 && most * tab.M > BLUE_HOLD * 256) most >>= 1;
@@ -408,7 +410,7 @@ bool blue_launch(int op, bool inv, const LineArgs& la, hipStream_t stream, int* 
             return true;
         }
     }
-    hipLaunchKernelGGL(blue_kernel, dim3(grid), dim3(block), lds, stream, ba);
+    hipLaunchKernelGGL(blue_kernel, grid, dim3(block), lds, stream, ba);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) *rc = fail(SFA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
     return true;

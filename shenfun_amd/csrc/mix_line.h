@@ -102,8 +102,9 @@ __global__ void __launch_bounds__(256) mix_kernel(MixArgs a)
 {
     const int tid = threadIdx.x, nth = blockDim.x;
     const int64_t ntile = (a.d2 + a.T - 1) / a.T;
-    const int64_t i1 = blockIdx.x / ntile;
-    const int64_t t0 = (blockIdx.x - i1 * ntile) * a.T;
+    const int64_t blk = wide_block(), i1 = blk / ntile;
+    if (i1 >= a.d1) return;
+    const int64_t t0 = (blk - i1 * ntile) * a.T;
     const MixPlan& pl = a.plan;
     MixTile m;
     m.T = a.T;
@@ -329,7 +330,7 @@ __global__ void __launch_bounds__(256) mix_kernel(MixArgs a)
 // 15.8 -> 8.9, 64 x 360 x 64 33.3 -> 13.7; R2C 180 x 150 x 200 42.2 -> 24.3,
 // 256 x 256 x 240 98.0 -> 51.7; DCT-II / DCT-III with stencil along axis 0
 // 192 x 96 x 81 34.2 / 38.1 -> 19.4 / 16.6, 256 x 256 x 129 162 / 186 -> 94 / 80.
-inline bool mix_setup(const LineArgs& la, MixArgs& a, unsigned* grid, unsigned* block, size_t* lds_bytes,
+inline bool mix_setup(const LineArgs& la, MixArgs& a, dim3* grid, unsigned* block, size_t* lds_bytes,
                       int most = 16)
 {
     const int nf = la.plan.nfft;
@@ -370,14 +371,13 @@ inline bool mix_setup(const LineArgs& la, MixArgs& a, unsigned* grid, unsigned* 
     const size_t lds = (size_t)(T * line + table) + (size_t)2 * T * sizeof(double2);
     if (lds > 160 * 1024) return false;
     const int64_t nblk = d1 * ((d2 + T - 1) / T);
-    if (nblk >= (1ll << 31)) return false;
     // a thread per butterfly of the pass that has the most, at most 256; all 256
     // where the workgroups are few, for the steps that go over elements
     int rmin = kMixMaxRadix;
     for (int l = 0; l < a.plan.np; ++l) rmin = a.plan.r[l] < rmin ? a.plan.r[l] : rmin;
     const int64_t nbf = (int64_t)T * nf / rmin;
     *block = nbf >= 256 || nblk < 64 ? 256u : (unsigned)((nbf + 63) / 64 * 64);
-    *grid = (unsigned)nblk;
+    *grid = wide_grid(nblk);
     *lds_bytes = lds;
     return true;
 }
@@ -409,7 +409,8 @@ bool blue_launch(int op, bool inv, const LineArgs& la, hipStream_t stream, int* 
 inline bool mix_launch(int op, bool inv, const LineArgs& la, hipStream_t stream, int* rc)
 {
     MixArgs a;
-    unsigned grid, block;
+    dim3 grid;
+    unsigned block;
     size_t lds;
     if (!mix_setup(la, a, &grid, &block, &lds)) return blue_launch(op, inv, la, stream, rc);
     const bool c = la.in_cplx != 0;

@@ -49,8 +49,9 @@ __global__ void __launch_bounds__(256) line_kernel(LineArgs a)
     extern __shared__ double2 smem[];
     const int tid = threadIdx.x, nth = blockDim.x;
     const int64_t ntile = (a.d2 + a.T - 1) / a.T;
-    const int64_t i1 = blockIdx.x / ntile;
-    const int64_t t0 = (blockIdx.x - i1 * ntile) * a.T;
+    const int64_t blk = wide_block(), i1 = blk / ntile;
+    if (i1 >= a.d1) return;
+    const int64_t t0 = (blk - i1 * ntile) * a.T;
     const int T = a.T;
     const int Tv = (int)((a.d2 - t0) < T ? (a.d2 - t0) : T);  // valid lines in this tile
     const int ldn = a.ldn;
@@ -329,8 +330,7 @@ static int launch_line(int op, bool inv, LineArgs& a, hipStream_t stream)
     SFA_CHECK(lds <= 160 * 1024, SFA_ERR_UNSUPPORTED, "transform length %d too large for LDS", a.n);
     const int64_t ntile = (a.d2 + a.T - 1) / a.T;
     const int64_t nblk = ntile * a.d1;
-    SFA_CHECK(nblk < (1ll << 31), SFA_ERR_UNSUPPORTED, "too many lines");
-    dim3 grid((unsigned)nblk), block(256);
+    const dim3 grid = wide_grid(nblk), block(256);
 #define SFA_LK(OPV, INVV)                                                                     \
     do {                                                                                     \
         auto kfn = line_kernel<OPV, INVV>;                                                   \

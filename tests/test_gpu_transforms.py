@@ -405,3 +405,21 @@ def test_large_prime_lines(sfa, n, layout):
                     np.moveaxis(z, layout, 0)[N - 2:] = 0
                 assert rel(V.backward(dev(z), kind="fast"),
                            S.basis_backward("chebyshev", bc, z, layout, quad=quad)) < TOL
+
+
+@pytest.mark.parametrize("n", [6, 17])
+def test_line_counts_past_one_grid(sfa, n):
+    """Lines whose workgroups hold 2^32 threads and more, more than one dimension
+    of a launch may have (a trailing dimension of 1: a workgroup per line),
+    by the mixed-radix form and by Bluestein's algorithm.  The lines repeat 64
+    different ones."""
+    print(f"[line counts past one grid n={n}]", flush=True)
+    from shenfun_amd import _lib
+    reps = (1 << 20) + 1  # 64 threads a line
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((64, n)) + 1j * rng.standard_normal((64, n))
+    u = dev(x).repeat(reps, 1).view(64 * reps, n, 1)
+    _lib.call("sfa_fft_c2c", _lib.ptr(u), _lib.ptr(u), 3, _lib.arr(u.shape), _lib.arr(u.stride()),
+              _lib.arr(u.stride()), 1, -1, 1.0, _lib.stream_ptr())
+    r = dev(np.fft.fft(x, axis=1))
+    assert float((u.view(reps, 64, n) - r).abs().amax()) < TOL * float(r.abs().max())
