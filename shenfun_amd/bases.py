@@ -645,7 +645,8 @@ class _PolyBase(SpectralBase):
         out = self.scalar_product(input_array, output_array, kind)
         if self.is_composite:
             solver = self._mass_solver()
-            if not self.has_nonhomogeneous_bcs and solver.solve_fn == "sfa_tdma_solve":
+            if not self.has_nonhomogeneous_bcs and solver.solve_fn == "sfa_tdma_solve" \
+                    and solver._hip_solve():
                 # zero boundary slots and the solve in one launch
                 lu = solver.perform_lu(out.device)
                 shp, st = _geom(out)

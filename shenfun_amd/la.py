@@ -17,7 +17,10 @@ import torch
 
 from . import _lib
 from .matrices import SparseMatrix, TPMatrix, _split_bc, apply_bc_matrices
-from .optimization import optimizer, runtimeoptimizer
+from .optimization import BACKENDS, optimizer, runtimeoptimizer
+
+
+_HIP = BACKENDS["hip"]
 
 
 def _no_host(*args, **kwargs):
@@ -131,6 +134,13 @@ class _Banded:
 
     # solves go through the static Solve resolved by the backend dispatch
     _dispatch = True
+
+    @classmethod
+    def _hip_solve(cls):
+        """Whether Solve resolves to the HIP backend's own function, which a
+        launch that does more at once may stand for."""
+        f = getattr(getattr(cls, "Solve", None), "resolved", None)
+        return f is not None and f.__module__ == _HIP
 
     def __call__(self, b, u=None, axis=0, constraints=()):
         u = _prepare(b, u)
@@ -439,10 +449,11 @@ class SolverGeneric1ND:
         u = _prepare(b, u)
         data = self.perform_lu(u.device)
         # mode 0 (index 0 along every non-axis dim) has factors of its own only
-        # where a constraint replaced its first row; the others' launch holds
-        # the same ones otherwise
+        # where a constraint replaced its first row, and a solve of its own only
+        # where another backend's Solve takes it; the others' launch holds the
+        # same ones otherwise
         own0 = len(constraints) > 0 or self.sol0._pinned or self._band is not None \
-            or self.kind == "threedma"
+            or self.kind == "threedma" or not self.sol0._hip_solve()
         if own0:
             s = [0] * u.dim()
             s[ax] = slice(None)

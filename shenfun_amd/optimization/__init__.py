@@ -46,6 +46,7 @@ def optimizer(func, wrap=True):
     @wraps(func)
     def wrapped_function(*args, **kwargs):
         return fun(*args, **kwargs)
+    wrapped_function.resolved = fun
     return wrapped_function
 
 

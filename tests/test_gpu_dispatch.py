@@ -198,3 +198,27 @@ def test_threedma_compat_class(sfa):
     assert rel(u, S.threedma_solve(b, data, 0, compat=True)) < 1e-13
     u = sfa.la.ThreeDMA(M)(torch.from_numpy(b.copy()).cuda())
     assert rel(u, np.linalg.solve(S.dense(d, n), b)) < 1e-12
+
+
+@pytest.mark.parametrize("bc", ["D", "N"])
+def test_other_backend_solve_is_reached(sfa, hip, monkeypatch, bc):
+    """forward() of a composite space and mode 0 of SolverGeneric1ND solve with
+    what TDMA.Solve resolves to: a fused launch takes its place only for the
+    HIP backend's own function."""
+    T = sfa.TensorProductSpace(None, (sfa.FunctionSpace(24, "legendre", bc=bc),
+                                      sfa.FunctionSpace(16, "F", dtype="d")))
+    H = sfa.la.SolverGeneric1ND(sfa.helmholtz_tpmatrices(T, 2.0))
+    f = torch.randn((24, 16), dtype=torch.float64, device="cuda")
+    want = T.forward(f, sfa.Function(T)).clone()
+    b = T.scalar_product(f, sfa.Function(T))
+    sol = H(b.clone(), sfa.Function(T)).clone()
+    shapes = []
+
+    def solve(u, data, axis):
+        shapes.append(tuple(u.shape))
+        return hip.TDMA_Solve(u, data, axis)
+    monkeypatch.setattr(sfa.la.TDMA, "Solve", staticmethod(solve))
+    assert rel(T.forward(f, sfa.Function(T)), want.cpu().numpy()) < 1e-15
+    assert shapes == [(24, 9)]
+    assert rel(H(b.clone(), sfa.Function(T)), sol.cpu().numpy()) < 1e-13
+    assert len(shapes) == 2
