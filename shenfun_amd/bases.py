@@ -354,28 +354,28 @@ class _PolyBase(SpectralBase):
         """Whether the transform of this kind is a dense contraction."""
         return True
 
-    @staticmethod
-    def _padded_dense(twin, kind, inp, out):
-        # (arrays of one storage may overlap: those go through a temporary)
-        return twin._dense(kind, inp, out) and \
+    def _padded_dense(self, twin, kind, inp, out):
+        # (arrays of one storage may overlap: those go through a temporary; so
+        # do padded lengths below N, which the padding refuses)
+        return twin.N >= self.N and twin._dense(kind, inp, out) and \
             inp.untyped_storage().data_ptr() != out.untyped_storage().data_ptr()
 
     def _padded_matrix(self, which, twin):
         """The padded-length twin's analysis rows ('a') or synthesis columns
-        ('s') of this space's own functions, zero for the boundary slots: the
-        padding or truncation of the coefficients inside the product."""
+        ('s') of this space's own functions: the padding or truncation of the
+        coefficients inside the product."""
         key = ("padded", which)
         if key not in self._cache:
             n = self.dim()
-            if which == "a":
-                M = torch.zeros((self.N, twin.N), dtype=torch.float64, device=self.device)
-                M[:n] = twin._analysis_matrix()[:n]
-            else:
-                M = torch.zeros((twin.N, self.N), dtype=torch.float64, device=self.device)
-                M[:, :n] = twin._synthesis_matrix()[:, :n]
+            M = twin._analysis_matrix()[:n] if which == "a" else twin._synthesis_matrix()[:, :n]
+            M = M.contiguous()
             torch.cuda.current_stream(M.device).synchronize()  # other streams may take it from the cache
             self._cache[key] = M
         return self._cache[key]
+
+    def _own(self, t):
+        """The rows of this space's own functions (all but the boundary slots)."""
+        return t.narrow(self.axis, 0, self.dim())
 
     # ------------------------------------------------------------ transforms
     def _clone(self, N, padding_factor=1, dealias_direct=False):
@@ -579,6 +579,10 @@ class _PolyBase(SpectralBase):
         return t
 
     def scalar_product(self, input_array=None, output_array=None, kind=None):
+        return self._project(input_array, output_array, kind, True)
+
+    def _project(self, input_array, output_array, kind, slots):
+        # slots False: the caller writes the boundary slots of a padded space
         kind = self._kind(kind)
         inp = self._tensor(input_array)
         _check(inp, "input_array")
@@ -590,7 +594,9 @@ class _PolyBase(SpectralBase):
             # (spectralbase.py:225-229, _truncation_forward :1362-1366)
             twin = self._twin()
             if self._padded_dense(twin, kind, inp, out):  # the kept rows of its matrix, in one product
-                self._matmul(inp, out, self._padded_matrix("a", twin), 1)
+                self._matmul(inp, self._own(out), self._padded_matrix("a", twin), 1)
+                if slots and self.dim() < self.N:
+                    out.narrow(self.axis, self.dim(), self.N - self.dim()).zero_()
                 return out
             tmp = self._tmp("sp", inp.shape, inp.dtype)
             twin._scalar_product(inp, tmp, kind)
@@ -616,7 +622,7 @@ class _PolyBase(SpectralBase):
             # padded-length synthesis
             twin = self._twin()
             if self._padded_dense(twin, kind, inp, out):
-                self._matmul(inp, out, self._padded_matrix("s", twin), 2)
+                self._matmul(self._own(inp), out, self._padded_matrix("s", twin), 2)
             else:
                 shp = list(inp.shape)
                 shp[self.axis] = self._phys_len()
@@ -642,7 +648,7 @@ class _PolyBase(SpectralBase):
         (spectralbase.py:235-263, apply_inverse_mass :560-577).  BC slots
         N-2, N-1 of a composite space are set to 0 (homogeneous BCs,
         tensorproductspace.py:2091-2106)."""
-        out = self.scalar_product(input_array, output_array, kind)
+        out = self._project(input_array, output_array, kind, False)
         if self.is_composite:
             solver = self._mass_solver()
             if not self.has_nonhomogeneous_bcs and solver.solve_fn == "sfa_tdma_solve" \
@@ -1282,7 +1288,7 @@ class _StencilSpace:
             return super().forward(input_array, output_array, kind)
         if self.kind in ("P2", "P4"):
             raise NotImplementedError(f"{self.kind} is a test space: scalar_product and backward only")
-        out = self.scalar_product(input_array, output_array, kind)
+        out = self._project(input_array, output_array, kind, False)
         sl = [slice(None)] * out.dim()
         sl[self.axis] = slice(self.dim(), self.N)
         out[tuple(sl)] = 0

@@ -220,3 +220,41 @@ def test_padded_stencil_spaces(sfa, fam, bc):
     lo = V._direct_range()[0]
     cz[lo:V.dim()] = 0
     assert rel(D.backward(c), V.backward(cz).cpu().numpy()) < 1e-12
+
+
+@pytest.mark.parametrize("fam,bc", [("C", "D"), ("L", "N"), ("L", "DN"), ("C", "Biharmonic"), ("L", None)])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_padded_dense_boundary_slots(sfa, fam, bc, axis):
+    """Padded dense transforms neither read nor compute the boundary slots: a
+    NaN there stays out of backward, one in the data out of the scalar
+    product's slots (plain zeros); forward takes arrays that held anything."""
+    print(f"[padded slots {fam} {bc} axis={axis}]", flush=True)
+    N = 40
+    bcs = {"DN": {"left": {"D": 0}, "right": {"N": 0}}, "Biharmonic": (0, 0, 0, 0)}.get(bc, bc)
+    P = sfa.FunctionSpace(N, fam, bc=bcs).get_dealiased(1.5)
+    P.axis, P.dimensions = axis, 3
+    n = P.dim()
+    rng = np.random.default_rng(3)
+    shp = [3, 5, 7]
+    shp[axis] = N
+    c = dev(rng.standard_normal(shp))
+    c.narrow(axis, n, N - n).zero_()
+    d = c.clone()
+    d.narrow(axis, n, N - n).fill_(np.nan)
+    u = P.backward(c).clone()  # (a space returns its own output array)
+    assert bool(torch.isfinite(u).all()) and torch.equal(P.backward(d), u)
+    nan = torch.full(shp, np.nan, dtype=torch.float64, device="cuda")
+    want = P.scalar_product(u).clone()
+    assert not bool(want.narrow(axis, n, N - n).any())
+    assert torch.equal(P.scalar_product(u, nan), want)
+    want = P.forward(u).clone()
+    assert torch.equal(P.forward(u, torch.full_like(nan, np.nan)), want)
+    u.select(axis, 1)[0] = np.nan
+    s = P.scalar_product(u)
+    assert not bool(s.narrow(axis, n, N - n).any())
+    assert bool(torch.isnan(s.narrow(axis, 0, n)).any())
+    if n < N:  # a padded length between the functions and the points: refused
+        Q = sfa.FunctionSpace(N, fam, bc=bcs).get_dealiased((n + 0.5) / N)
+        Q.axis, Q.dimensions = axis, 3
+        with pytest.raises(RuntimeError):
+            Q.scalar_product(u.narrow(axis, 0, n).contiguous())
