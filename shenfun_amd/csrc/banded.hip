@@ -484,11 +484,27 @@ __global__ void poisson_add_kernel(const T* __restrict__ b, T* __restrict__ u, L
 // shared factors 51.5 -> 17.1 us, 512 x 129 with factors per line, mode 0 in a
 // launch of its own, 194 + 123 -> 7.8 us in one.
 //
-// A segment's factor is kept within +-kChainMax: a product of multipliers that
-// overflowed would turn a line of zeros into NaN, where row by row it stays
-// zero (a state that is not zero overflows either way).
-constexpr double kChainMax = 1e300;
-__device__ inline double chain_clamp(double a) { return fmin(fmax(a, -kChainMax), kChainMax); }
+// The maps' factors are kept as a number times a power of two: a product of
+// multipliers may pass the largest double, or fall below the smallest, where the
+// values themselves, row by row, stay in range (and a line of zeros stays zero).
+// A segment's factor is split once, after its rows (at most 8 multipliers); the
+// numbers of products over the at most 256 segments then stay far inside the
+// range.  Against plain doubles a solve of few lines takes 0.3 us (TDMA) and 0.9 us
+// (Helmholtz) more, one bound by its bytes the same.
+struct ChainFac {
+    double a;
+    int e;  // times 2^e
+};
+__device__ inline ChainFac chain_fac(double a, int e = 0)  // a in [1/2, 1) or 0
+{
+    return ChainFac{__builtin_amdgcn_frexp_mant(a), e + __builtin_amdgcn_frexp_exp(a)};
+}
+__device__ inline ChainFac chain_mul(ChainFac f, ChainFac g) { return ChainFac{f.a * g.a, f.e + g.e}; }
+__device__ inline ChainFac chain_add(ChainFac f, ChainFac g)
+{
+    const int e = f.a == 0.0 ? g.e : g.a == 0.0 ? f.e : f.e > g.e ? f.e : g.e;
+    return chain_fac(ldexp(f.a, f.e - e) + ldexp(g.a, g.e - e), e);
+}
 
 template <typename T>
 struct ChainArgs {
@@ -511,16 +527,24 @@ __device__ inline double shflu(double v, int d) { return __shfl_up(v, d); }
 __device__ inline double2 shflu(double2 v, int d) { return make_double2(__shfl_up(v.x, d), __shfl_up(v.y, d)); }
 __device__ inline double shfld(double v, int d) { return __shfl_down(v, d); }
 __device__ inline double2 shfld(double2 v, int d) { return make_double2(__shfl_down(v.x, d), __shfl_down(v.y, d)); }
+__device__ inline double ldx(double a, int e) { return ldexp(a, e); }
+__device__ inline double2 ldx(double2 a, int e) { return make_double2(ldexp(a.x, e), ldexp(a.y, e)); }
 __device__ inline double axpb(double a, double x, double b) { return a * x + b; }
 __device__ inline double2 axpb(double a, double2 x, double2 b) { return make_double2(a * x.x + b.x, a * x.y + b.y); }
+template <typename T>
+__device__ inline T axpb(ChainFac f, T x, T b)
+{
+    return add(ldx(mul(x, f.a), f.e), b);
+}
 
 template <typename T, int TL, int E, bool HELM, bool ONE>
 __global__ void __launch_bounds__(256) chain_solve_kernel(ChainArgs<T> g)
 {
     constexpr int SG = 256 / TL, WS = 64 / TL, NW = 4;
-    __shared__ double sA[NW][TL];
+    __shared__ ChainFac sA[NW][TL], sF[NW][TL];  // forward, backward (no barrier lies between them)
     __shared__ T sB[NW][TL];
-    __shared__ double sM[NW][TL][HELM ? 4 : 1];
+    __shared__ double sM[NW][TL][HELM ? 3 : 1];
+    __shared__ int sE[NW][TL];
     __shared__ T sC[NW][TL][2];
     const int tid = threadIdx.x, t = tid % TL, seg = tid / TL, wave = tid >> 6, ws = seg % WS;
     const int p = blockIdx.y, n = g.n;
@@ -577,26 +601,27 @@ __global__ void __launch_bounds__(256) chain_solve_kernel(ChainArgs<T> g)
             am[e] = in && m > 0 ? -lo[(int64_t)(p + 2 * m - 2) * sf] : 0.0;
         }
         if (ONE) load_back(m0);
-        double A = 1.0;
+        double A0 = 1.0;
         T B = zero<T>();
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             B = axpb(am[e], B, y[e]);
-            A = chain_clamp(A * am[e]);
+            A0 *= am[e];
         }
+        ChainFac A = chain_fac(A0);
 #pragma unroll
         for (int k = 1; k < WS; k <<= 1) {
-            const double oA = shflu(A, TL * k);
+            const ChainFac oA{shflu(A.a, TL * k), __shfl_up(A.e, TL * k)};
             const T oB = shflu(B, TL * k);
             if (ws >= k) {
                 B = axpb(A, oB, B);
-                A = chain_clamp(A * oA);
+                A = chain_mul(A, oA);
             }
         }
-        double eA = shflu(A, TL);
+        ChainFac eA{shflu(A.a, TL), __shfl_up(A.e, TL)};
         T eB = shflu(B, TL);
         if (ws == 0) {
-            eA = 1.0;
+            eA = ChainFac{1.0, 0};
             eB = zero<T>();
         }
         if (ws == WS - 1) {
@@ -635,7 +660,18 @@ __global__ void __launch_bounds__(256) chain_solve_kernel(ChainArgs<T> g)
         }
         const double d00 = iv[0];
         T Bx = zero<T>(), Bs = zero<T>();
-        double M00 = 1.0, M01 = 0.0, M10 = 0.0, M11 = 1.0;  // TDMA: M00 alone
+        // the segment's map: x from x by F, the other three of the 2 x 2 matrix
+        // (Helmholtz) times 2^Me.  F keeps its own exponent: beside M10 >= 1
+        // (the sum takes x as it is) it may be below the smallest double.
+        double M00 = 1.0, M01 = 0.0, M10 = 0.0, M11 = 1.0;
+        int Me = 0;
+        auto scaled = [&]() {  // the largest of the three in [1/2, 1)
+            const int ex = __builtin_amdgcn_frexp_exp(fmax(fabs(M01), fmax(fabs(M10), fabs(M11))));
+            M01 = ldexp(M01, -ex);
+            M10 = ldexp(M10, -ex);
+            M11 = ldexp(M11, -ex);
+            Me += ex;
+        };
 #pragma unroll
         for (int e = E - 1; e >= 0; --e) {
             const bool in = valid && m0 + e < K;
@@ -654,52 +690,64 @@ __global__ void __launch_bounds__(256) chain_solve_kernel(ChainArgs<T> g)
                 M01 = n01;
             } else {
                 Bx = axpb(q[e], Bx, y[e]);
-                M00 = chain_clamp(M00 * q[e]);
+                M00 *= q[e];
             }
         }
+        ChainFac F = chain_fac(M00);
+        if constexpr (HELM) scaled();
 #pragma unroll
         for (int k = 1; k < WS; k <<= 1) {
-            const double o00 = shfld(M00, TL * k);
+            const ChainFac oF{shfld(F.a, TL * k), __shfl_down(F.e, TL * k)};
             const T ox = shfld(Bx, TL * k);
             if constexpr (HELM) {
                 const double o01 = shfld(M01, TL * k), o10 = shfld(M10, TL * k), o11 = shfld(M11, TL * k);
+                const int oe = __shfl_down(Me, TL * k);
                 const T os = shfld(Bs, TL * k);
                 if (ws + k < WS) {
-                    Bx = add(axpb(M00, ox, Bx), mul(os, M01));
-                    Bs = add(axpb(M10, ox, Bs), mul(os, M11));
-                    const double n00 = M00 * o00 + M01 * o10, n01 = M00 * o01 + M01 * o11;
+                    Bx = add(axpb(F, ox, Bx), ldx(mul(os, M01), Me));
+                    Bs = add(ldx(axpb(M10, ox, mul(os, M11)), Me), Bs);
+                    const double o00 = ldexp(oF.a, oF.e - oe), f00 = ldexp(F.a, F.e - Me);
+                    const double n01 = f00 * o01 + M01 * o11;
                     const double n10 = M10 * o00 + M11 * o10, n11 = M10 * o01 + M11 * o11;
-                    M00 = n00;
+                    F = chain_add(chain_mul(F, oF), chain_mul(ChainFac{M01, Me}, ChainFac{o10, oe}));
                     M01 = n01;
                     M10 = n10;
                     M11 = n11;
+                    Me += oe;
+                    scaled();
                 }
             } else if (ws + k < WS) {
-                Bx = axpb(M00, ox, Bx);
-                M00 = chain_clamp(M00 * o00);
+                Bx = axpb(F, ox, Bx);
+                F = chain_mul(F, oF);
             }
         }
         // the maps of the segments after this one in the wave
-        double e00 = shfld(M00, TL), e01 = 0.0, e10 = 0.0, e11 = 1.0;
+        ChainFac eF{shfld(F.a, TL), __shfl_down(F.e, TL)};
+        double e01 = 0.0, e10 = 0.0, e11 = 1.0;
+        int ee = 0;
         T ex = shfld(Bx, TL), es = zero<T>();
         if constexpr (HELM) {
             e01 = shfld(M01, TL);
             e10 = shfld(M10, TL);
             e11 = shfld(M11, TL);
+            ee = __shfl_down(Me, TL);
             es = shfld(Bs, TL);
         }
         if (ws == WS - 1) {
-            e00 = e11 = 1.0;
+            eF = ChainFac{1.0, 0};
+            e11 = 1.0;
             e01 = e10 = 0.0;
+            ee = 0;
             ex = es = zero<T>();
         }
         if (ws == 0) {
-            sM[wave][t][0] = M00;
+            sF[wave][t] = F;
             sC[wave][t][0] = Bx;
             if constexpr (HELM) {
-                sM[wave][t][1] = M01;
-                sM[wave][t][2] = M10;
-                sM[wave][t][3] = M11;
+                sE[wave][t] = Me;
+                sM[wave][t][0] = M01;
+                sM[wave][t][1] = M10;
+                sM[wave][t][2] = M11;
                 sC[wave][t][1] = Bs;
             }
         }
@@ -708,21 +756,21 @@ __global__ void __launch_bounds__(256) chain_solve_kernel(ChainArgs<T> g)
 #pragma unroll
         for (int k = NW - 1; k >= 0; --k) {
             if constexpr (HELM) {
-                const T nx = add(axpb(sM[k][t][0], cx, sC[k][t][0]), mul(cs, sM[k][t][1]));
-                cs = add(axpb(sM[k][t][2], cx, sC[k][t][1]), mul(cs, sM[k][t][3]));
+                const T nx = add(axpb(sF[k][t], cx, sC[k][t][0]), ldx(mul(cs, sM[k][t][0]), sE[k][t]));
+                cs = add(ldx(axpb(sM[k][t][1], cx, mul(cs, sM[k][t][2])), sE[k][t]), sC[k][t][1]);
                 cx = nx;
             } else {
-                cx = axpb(sM[k][t][0], cx, sC[k][t][0]);
+                cx = axpb(sF[k][t], cx, sC[k][t][0]);
             }
             if (k > wave) {
                 ix = cx;
                 is = cs;
             }
         }
-        T x = axpb(e00, ix, ex), s = zero<T>();
+        T x = axpb(eF, ix, ex), s = zero<T>();
         if constexpr (HELM) {
-            x = add(x, mul(is, e01));
-            s = add(axpb(e10, ix, es), mul(is, e11));
+            x = add(x, ldx(mul(is, e01), ee));
+            s = add(ldx(axpb(e10, ix, mul(is, e11)), ee), es);
         }
 #pragma unroll
         for (int e = E - 1; e >= 0; --e) {

@@ -384,3 +384,51 @@ def test_solve_line_counts_past_one_grid(sfa, kind):
     u = u.view(reps, 64, N)[:, :, :n]
     r = dev(np.ascontiguousarray(ref[:, :n]))
     assert float((u - r).abs_().amax()) < TOL * float(r.abs().max())
+
+
+@pytest.mark.parametrize("lines,axis", [(1, 0), (600, 0), (2050, 0), (5, 1), (2050, 1)])
+@pytest.mark.parametrize("solver", ["tdma", "helmholtz"])
+@pytest.mark.parametrize("sweep", ["forward", "backward"])
+def test_chain_scan_range(sfa, lines, axis, solver, sweep):
+    """One value per chain carried over 1,000 rows by multipliers whose product
+    over a wave's rows (256, 128 or 32 of them) leaves the range of a double in
+    either direction, while the values never do.  All of it is powers of two,
+    so the result is exact row by row."""
+    print(f"[chain range {solver} {sweep} lines={lines} axis={axis}]", flush=True)
+    from shenfun_amd import _lib
+    n = 2000
+    K = n // 2
+    for g, sign in ((4, 1), (8, 1), (33, 1), (4, -1), (8, -1), (33, -1)):
+        # x_m = -2^steps[m-1] x_{m-1} along the sweep: level, 2^2000 up (or
+        # down) from the first row of a wave on, level
+        m0 = 255 if sweep == "forward" else 231
+        steps = np.zeros(K - 1, dtype=int)
+        steps[m0:m0 + 2000 // g] = g * sign
+        ex = -1000 * sign + np.concatenate([[0], np.cumsum(steps)])
+        x = np.ldexp((-1.0) ** np.arange(K), ex)
+        mult = np.ldexp(1.0, steps)
+        if sweep == "backward":
+            x, mult = x[::-1], mult[::-1]
+        start = 0 if sweep == "forward" else K - 1
+        ref, rhs = np.repeat(x, 2)[None, :], np.zeros((1, n))  # rows 2 m and 2 m + 1 alike
+        rhs[0, [2 * start, 2 * start + 1]] = x[start]
+        sc = np.ldexp(1.0, np.arange(lines) % 4)[:, None]
+        ref, rhs = sc * ref, sc * rhs
+        m2 = np.repeat(mult, 2)
+        z = np.zeros(n)
+        lo, hi = (m2, 0 * m2) if sweep == "forward" else (0 * m2, m2)
+        N = n + 2 if solver == "helmholtz" else n
+        b = np.zeros((lines, N))
+        b[:, :n] = rhs
+        u = dev(b if axis == 1 else b.T)
+        shp, st = _lib.arr(u.shape), _lib.arr(u.stride())
+        if solver == "tdma":
+            d = dev(np.stack([np.append(lo, [0, 0]), np.ones(n), np.append([0, 0], hi)]))
+            _lib.call("sfa_tdma_solve", _lib.ptr(u), _lib.F64, 2, shp, st, axis, _lib.ptr(d), n, 0, 0,
+                      _lib.stream_ptr())
+        else:
+            f = [dev(np.append(v, np.zeros(N - v.size))) for v in (np.ones(N), hi, z, lo)]
+            _lib.call("sfa_helmholtz_solve", _lib.ptr(u), _lib.ptr(u), _lib.F64, 2, shp, st, st, axis, 0,
+                      *[_lib.ptr(v) for v in f], _lib.arr((0, 1) if axis == 1 else (1, 0)), _lib.stream_ptr())
+        got = u.cpu().numpy() if axis == 1 else u.cpu().numpy().T
+        assert np.max(np.abs(got[:, :n] / ref - 1.0)) < 1e-12
