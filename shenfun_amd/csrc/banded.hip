@@ -470,7 +470,7 @@ __global__ void poisson_add_kernel(const T* __restrict__ b, T* __restrict__ u, L
 // it runs its rows once more.  Bound: a thread per chain waits for memory once
 // per row with too few waves to hide it (8,320 lines of 63 rows at 128^3 are
 // 260 waves on 1,024 SIMDs); here all of a thread's rows are loaded before the
-// first of them is used and a chain is spread over 16 to 256 threads.
+// first of them is used and a chain is spread over 4 to 256 threads.
 //
 // A workgroup has TL lines x 256 / TL segments, a line's segments TL lanes
 // apart, so that lanes run over lines (coalesced where the lines are
@@ -797,33 +797,72 @@ __global__ void __launch_bounds__(256) chain_solve_kernel(ChainArgs<T> g)
     }
 }
 
-template <typename T, int TL, bool HELM>
+template <int TL, int E, bool ONE, bool HELM, typename T>
+static void chain_run(const ChainArgs<T>& a, hipStream_t s)
+{
+    hipLaunchKernelGGL((chain_solve_kernel<T, TL, E, HELM, ONE>), wide_grid((a.gu.nlines + TL - 1) / TL, 2),
+                       dim3(256), 0, s, a);
+}
+
+// The fewest rows per thread that hold the chain in one chunk, of those that
+// chain_tl's choice of TL can meet.
+template <int TL, bool HELM, typename T>
 static void chain_launch_tl(const ChainArgs<T>& a, hipStream_t s)
 {
     constexpr int SG = 256 / TL;
     const int K = (a.n + 1) / 2;
-    const dim3 grid = wide_grid((a.gu.nlines + TL - 1) / TL, 2), block(256);
-    if (K <= SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 1, HELM, true>), grid, block, 0, s, a);
-    else if (K <= 2 * SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 2, HELM, true>), grid, block, 0, s, a);
-    else if (K <= 4 * SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 4, HELM, true>), grid, block, 0, s, a);
-    else if (K <= 8 * SG) hipLaunchKernelGGL((chain_solve_kernel<T, TL, 8, HELM, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((chain_solve_kernel<T, TL, 8, HELM, false>), grid, block, 0, s, a);
+    if constexpr (TL == 1 || TL == 16)
+        if (K <= SG) return chain_run<TL, 1, true, HELM>(a, s);
+    if (K <= 2 * SG) return chain_run<TL, 2, true, HELM>(a, s);
+    if (K <= 4 * SG) return chain_run<TL, 4, true, HELM>(a, s);
+    if constexpr (TL == 8 || TL == 16)
+        if (K <= 6 * SG) return chain_run<TL, 6, true, HELM>(a, s);
+    if (K <= 8 * SG) return chain_run<TL, 8, true, HELM>(a, s);
+    chain_run<TL, 8, false, HELM>(a, s);
 }
 
-// Lines per workgroup: 16 (256-byte row segments of complex lines) where that
-// still gives every compute unit a workgroup, 2048 lines being 256 of them; else
-// 4, then 1, and as many more segments per chain: below 512 lines of up to 2048
-// rows the arrays are a few MB and latency is the cost, so a chain goes over all
-// 256 threads.  1 also where the axis is the contiguous one (the lanes of a wave
-// then read one line).
+// Lines per workgroup for chains of K rows.  At least as many as leave a thread
+// one or two of its 256 / TL share of the rows (a chain of 7 rows over 256 threads
+// takes as long as one of 511), at most as many as hold the chain in one chunk of
+// 8 rows a thread, and between the two by the number of lines, so that at least
+// 128 workgroups of each parity are in flight.
+//   Lines side by side in memory (complex, TDMA / Helmholtz, microseconds; TL by
+//   this rule | 16, 4 or 1 by the number of lines alone | a thread per chain):
+//   14 rows x 131072 lines 13.6/24.1 | 42.9/70.2 | 10.5/24.2, 62 x 32768 12.0/25.4 |
+//   17.4/28.4 | 17.8/32.3, 254 x 8192 15.3/24.7 in both | 53/94, 510 x 32768 98/288 |
+//   145/289 | 177/370.  From 65536 lines on chains beyond one chunk of 16 lines go
+//   64 lines wide (1022 x 131072: 1542/2458, 16 wide 1656/2735, thread per chain
+//   1569/2488); reals, half as wide in bytes, take 16 lines where 8 hold a chunk
+//   (510 x 8192 47, 8 lines 59).
+//   Lines along memory: a thread's two rows share its cache line with its
+//   neighbours', so the smallest count is the best one (62 x 32768 22.5/48.3, 1
+//   line per workgroup 300/518, a thread per chain 33/73; 254 x 32768 103/247,
+//   306/520, 146/403; 510 x 131072 938/2193, 1228/2232, 2731/7762); up to 128 of
+//   them are spread over the chip instead (254 x 16: 4.2/5.9 against 4.8/6.3).
+static int chain_tl(int K, int64_t nlines, bool across, bool cplx)
+{
+    const int least = K <= 8 ? 64 : K <= 32 ? 16 : K <= 64 ? 8 : K <= 256 ? 4 : 1;
+    if (!across) return K > 32 && nlines <= 128 ? 1 : least;
+    if (K > 128 && nlines >= 65536) return 64;
+    if (K > 256) return nlines < 128 ? 1 : nlines < 2048 ? 4 : 16;
+    const int most = K <= 32 ? 64 : K <= 128 || !cplx ? 16 : 8;
+    const int fill = nlines >= 8192 ? 64 : nlines >= 2048 ? 16 : nlines >= 1024 ? 8 : 4;
+    const int tl = fill < most ? fill : most;
+    return tl > least ? tl : least;
+}
+
 template <typename T, bool HELM>
 static void chain_launch(const ChainArgs<T>& a, hipStream_t s)
 {
     auto absl = [](int64_t v) { return v < 0 ? -v : v; };
     const bool across = absl(a.gu.s2) < absl(a.gu.sa) && a.gu.d2 > 1;
-    if (across && a.gu.nlines >= 2048) chain_launch_tl<T, 16, HELM>(a, s);
-    else if (across && a.gu.nlines >= 512) chain_launch_tl<T, 4, HELM>(a, s);
-    else chain_launch_tl<T, 1, HELM>(a, s);
+    switch (chain_tl((a.n + 1) / 2, a.gu.nlines, across, sizeof(T) == 16)) {
+        case 64: return chain_launch_tl<64, HELM>(a, s);
+        case 16: return chain_launch_tl<16, HELM>(a, s);
+        case 8: return chain_launch_tl<8, HELM>(a, s);
+        case 4: return chain_launch_tl<4, HELM>(a, s);
+        default: return chain_launch_tl<1, HELM>(a, s);
+    }
 }
 
 // ----------------------------------------------------------------- host

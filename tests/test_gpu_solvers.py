@@ -432,3 +432,45 @@ def test_chain_scan_range(sfa, lines, axis, solver, sweep):
                       *[_lib.ptr(v) for v in f], _lib.arr((0, 1) if axis == 1 else (1, 0)), _lib.stream_ptr())
         got = u.cpu().numpy() if axis == 1 else u.cpu().numpy().T
         assert np.max(np.abs(got[:, :n] / ref - 1.0)) < 1e-12
+
+
+@pytest.mark.parametrize("N,lines,axis", [
+    (10, 300, 0), (18, 8201, 0), (19, 8192, 0), (34, 8250, 0), (35, 2050, 0), (66, 8201, 0),  # 64, 16
+    (67, 1030, 0), (130, 1500, 0), (131, 600, 0), (194, 2050, 0), (196, 2049, 0), (258, 2100, 0),  # 8, 4, 16
+    (260, 1100, 0), (386, 2048, 0), (388, 2050, 0), (514, 2050, 0), (516, 130, 0), (516, 2050, 0),  # 8, 16 (reals), 4
+    (260, 65540, 0), (516, 65600, 0),  # 64, several chunks
+    (10, 2051, 1), (18, 40, 1), (34, 2050, 1), (66, 2050, 1), (67, 129, 1), (67, 128, 1), (130, 2050, 1),
+    (258, 2050, 1), (514, 2050, 1), (516, 2050, 1)])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_chain_scan_lines_per_workgroup(sfa, N, lines, axis, cplx):
+    """Every number of lines per workgroup and rows per thread that the solves
+    choose between, at and one past the limits of rows (K = (N - 1) // 2 for a
+    system of N - 2) and lines, across and along memory; 32 different lines,
+    repeated, vs the oracle."""
+    print(f"[chain lines N={N} lines={lines} axis={axis} cplx={cplx}]", flush=True)
+    from shenfun_amd import _lib
+    rng = np.random.default_rng(N + lines)
+    n = N - 2
+    b = rng.standard_normal((N, 32)) + (1j * rng.standard_normal((N, 32)) if cplx else 0.0)
+    d3 = {0: rng.uniform(2, 3, n), -2: rng.uniform(0.1, 1, n - 2), 2: rng.uniform(0.1, 1, n - 2)}
+    lu = S.tdma_lu(S.tdma_dia(d3, n))
+    fac = S.helmholtz_lu("D", N, -np.ones(1), np.full(1, 7.0))
+    idx = torch.arange(lines, device="cuda") % 32
+    code = _lib.C128 if cplx else _lib.F64
+    for kind in ("tdma", "helmholtz"):
+        u = dev(b)[:, idx].contiguous() if axis == 0 else dev(b.T)[idx].contiguous()
+        geom = (code, 2, _lib.arr(u.shape), _lib.arr(u.stride()))
+        if kind == "tdma":
+            ref = S.tdma_solve(b[:n], lu, 0)
+            lud = dev(lu)
+            _lib.call("sfa_tdma_mass_solve", _lib.ptr(u), *geom, axis, _lib.ptr(lud), n, 2, _lib.stream_ptr())
+        else:
+            ref = S.helmholtz_solve(b, *fac, neumann=False)[:n]
+            fd = [dev(x.reshape(-1)) for x in fac]
+            _lib.call("sfa_helmholtz_solve", _lib.ptr(u), _lib.ptr(u), *geom, _lib.arr(u.stride()), axis, 0,
+                      *[_lib.ptr(x) for x in fd], _lib.arr((1, 0) if axis == 0 else (0, 1)), _lib.stream_ptr())
+        got = u if axis == 0 else u.T
+        r = dev(ref)
+        assert float((got[:n] - r[:, idx]).abs().amax()) < TOL * float(r.abs().max())
+        if kind == "tdma":
+            assert not bool(got[n:].any())
