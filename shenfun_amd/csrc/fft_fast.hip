@@ -14,6 +14,13 @@ namespace sfa {
 
 constexpr int TL = 16;  // lines per block
 
+// Where a kernel lies in its code object moves its time by up to 2% at the same
+// instructions: the five of an FP64 256^3 solve took 268.3 us at one placement
+// and 269.9 at another, 1 KB on, that smaller kernels before them had led to (y
+// forward 46.0 and 46.5, C2R 43.9 and 44.9).  At multiples of 8 KB (or 16, 64):
+// 267.8; at 1 KB as fast, but the mixed 256^3 solve 0.5% slower.
+#define SFA_FFT_KERNEL __attribute__((aligned(8192))) __global__
+
 // ----------------------------------------------------------------- C2C strided
 struct StridedLines {
     const void* in;
@@ -58,7 +65,7 @@ __device__ __forceinline__ void c2c_strided_body(const StridedLines& g, const do
 }
 
 template <int N, bool INV, typename C2 = double2>
-__global__ void __launch_bounds__(TL * Pow2<N>::Q)
+SFA_FFT_KERNEL void __launch_bounds__(TL * Pow2<N>::Q)
     c2c_strided_kernel(StridedLines g, const double2* __restrict__ twg)
 {
     c2c_strided_body<N, INV, C2>(g, twg, blockIdx.x);
@@ -70,7 +77,7 @@ __global__ void __launch_bounds__(TL * Pow2<N>::Q)
 // (dispatched first) delivers the statistics in stats, which the previous
 // kernel finished, while the other blocks transform.
 template <int N, bool INV>
-__global__ void __launch_bounds__(TL * Pow2<N>::Q)
+SFA_FFT_KERNEL void __launch_bounds__(TL * Pow2<N>::Q)
     c2c_strided_dual_kernel(StridedLines g64, StridedLines g32, int64_t nblk64,
                             const double2* __restrict__ twg, const double* stats, StatOut out)
 {
@@ -157,7 +164,7 @@ __device__ __forceinline__ void r2c_contig_body(const double* __restrict__ in, d
 }
 
 template <int H>
-__global__ void __launch_bounds__(TL * Pow2<H>::Q)
+SFA_FFT_KERNEL void __launch_bounds__(TL * Pow2<H>::Q)
     r2c_contig_kernel(const double* __restrict__ in, double2* __restrict__ out, int64_t in_rs,
                       int64_t out_rs, int64_t d2, int64_t in_s1, int64_t out_s1, int64_t nrows,
                       double scale, const double2* __restrict__ twg /* 2H entries */)
@@ -260,7 +267,7 @@ __device__ __forceinline__ void c2r_contig_body(const double2* __restrict__ in, 
 }
 
 template <int H, bool ADD = false>
-__global__ void __launch_bounds__(TL * Pow2<H>::Q)
+SFA_FFT_KERNEL void __launch_bounds__(TL * Pow2<H>::Q)
     c2r_contig_kernel(const double2* __restrict__ in, double* __restrict__ out, int64_t in_rs,
                       int64_t out_rs, int64_t d2, int64_t in_s1, int64_t out_s1, int64_t nrows,
                       double scale, const double2* __restrict__ twg /* 2H entries */,
@@ -756,7 +763,7 @@ constexpr int xpass_minb() { return N >= 512 ? 1 : 2; }
 // FP64 x-pass.  NM: Neumann (Chebyshev SN) rows, else Dirichlet (SD); one
 // kernel each so that the Dirichlet kernels carry no Neumann code
 template <int N, bool NM>
-__global__ void __launch_bounds__(TL * Pow2<N>::Q, xpass_minb<N>()) xpass2_kernel(XPass2Args a)
+SFA_FFT_KERNEL void __launch_bounds__(TL * Pow2<N>::Q, xpass_minb<N>()) xpass2_kernel(XPass2Args a)
 {
     xpass2_body<N, double2, false, NM>(a, blockIdx.x);
 }
@@ -798,7 +805,7 @@ __device__ __forceinline__ int64_t xpass_pair_order(const XPass2Args& a, int64_t
 }
 
 template <int N, bool STATS, bool NM>
-__global__ void __launch_bounds__(TL * Pow2<N>::Q, xpass_minb<N>()) xpass2_dual_kernel(XPass2Args a64, XPass2Args a32,
+SFA_FFT_KERNEL void __launch_bounds__(TL * Pow2<N>::Q, xpass_minb<N>()) xpass2_dual_kernel(XPass2Args a64, XPass2Args a32,
                                                                         int64_t nb64)
 {
     const int64_t b = blockIdx.x;
@@ -985,7 +992,7 @@ __device__ __forceinline__ void r2c_split_body(const double* __restrict__ in, do
 // zero[0, nzero): cleared on the side (grid-stride), for the accumulators that
 // later kernels of the same pass add into, so no launch of its own is needed
 template <int H, bool KSMALL>
-__global__ void __launch_bounds__(TL * Pow2<H>::Q)
+SFA_FFT_KERNEL void __launch_bounds__(TL * Pow2<H>::Q)
     r2c_split_kernel(const double* __restrict__ in, double2* __restrict__ o64,
                      float2* __restrict__ o32, int64_t nrows, int Kh, double scale,
                      const double2* __restrict__ twg, double* __restrict__ zero, int nzero)
@@ -1084,7 +1091,7 @@ __device__ __forceinline__ void c2r_merge_body(const double2* __restrict__ i64, 
 }
 
 template <int H, bool KSMALL, bool ADD = false>
-__global__ void __launch_bounds__(TL * Pow2<H>::Q)
+SFA_FFT_KERNEL void __launch_bounds__(TL * Pow2<H>::Q)
     c2r_merge_kernel(const double2* __restrict__ i64, const float2* __restrict__ i32,
                      double* __restrict__ out, int64_t nrows, int Kh, double scale,
                      const double2* __restrict__ twg, const double* __restrict__ add, int64_t add_rows)
