@@ -423,3 +423,47 @@ def test_line_counts_past_one_grid(sfa, n):
               _lib.arr(u.stride()), 1, -1, 1.0, _lib.stream_ptr())
     r = dev(np.fft.fft(x, axis=1))
     assert float((u.view(reps, 64, n) - r).abs().amax()) < TOL * float(r.abs().max())
+
+
+@pytest.mark.parametrize("n", [6, 12, 17, 19, 34, 48, 100])
+@pytest.mark.parametrize("lines", [(5, 241), (41, 201)])
+@pytest.mark.parametrize("layout", [0, 1, 2])
+def test_short_lines_many(sfa, n, lines, layout):
+    """Short lines in thousands (workgroups of 64 to 256 threads, tiles of 8 and of
+    16 lines, the last one not full), by the mixed-radix form and by Bluestein's
+    algorithm: C2C in place, R2C / C2R at n and 2 n, both Chebyshev quadratures,
+    real and complex, with and without a stencil."""
+    print(f"[short lines n={n} lines={lines} layout={layout}]", flush=True)
+
+    def shp(k):
+        return ((k,) + lines, (lines[0], k, lines[1]), lines + (k,))[layout]
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(shp(n)) + 1j * rng.standard_normal(shp(n))
+    B = sfa.FunctionSpace(n, "F", dtype="D")
+    B.axis = layout
+    y = dev(x)
+    B.scalar_product(y, y)
+    assert rel(y, np.fft.fft(x, axis=layout) / n) < TOL
+    assert rel(B.backward(dev(x)), np.fft.ifft(x, axis=layout) * n) < TOL
+    for k in (n, 2 * n):
+        r = rng.standard_normal(shp(k))
+        R = sfa.FunctionSpace(k, "F", dtype="d")
+        R.axis = layout
+        c = np.fft.rfft(r, axis=layout)
+        assert rel(R.scalar_product(dev(r)), c / k) < TOL
+        assert rel(R.backward(dev(c)), r * k) < TOL
+    for bc in (None, "D", "N"):
+        for quad, N in (("GC", n), ("GL", n // 2 + 1)):  # GL: FFT length 2 (N - 1)
+            if N < 4:
+                continue
+            z0 = rng.standard_normal(shp(N)) + 1j * rng.standard_normal(shp(N))
+            for z in (z0, z0.real.copy()):
+                V = sfa.FunctionSpace(N, "chebyshev", bc=bc, quad=quad)
+                V.axis = layout
+                assert rel(V.scalar_product(dev(z), kind="fast"),
+                           S.basis_scalar_product("chebyshev", bc, z, layout, quad=quad)) < TOL
+                if bc is not None:
+                    z = z.copy()
+                    np.moveaxis(z, layout, 0)[N - 2:] = 0
+                assert rel(V.backward(dev(z), kind="fast"),
+                           S.basis_backward("chebyshev", bc, z, layout, quad=quad)) < TOL
