@@ -747,9 +747,10 @@ class ChebyshevBase(_PolyBase):
 
     # 'auto': up to this many points the transforms run as dense contractions
     # on FP64 MFMA (sfa_line_matmul_parity); above it as DCTs on the complex FFT
-    # kernels.  Measured on the MI355X along axis 0 of (N, N, N/2 + 1) arrays,
-    # scalar product / backward: N = 64 dense 8.2 / 8.6 us, DCT 10.5 / 8.8;
-    # N = 128 15.7 / 14.9 and 16.6 / 14.5; N = 256 132 / 115 and 98 / 84.
+    # kernels.  Measured on the MI355X along axis 0 of (N, N, N/2 + 1) arrays
+    # (GPU time, 20 calls in a graph), scalar product / backward: N = 64 dense
+    # 5.2 / 4.7 us, DCT 10.2 / 8.2; N = 128 15.8 / 15.0 and 16.3 / 14.2; N = 256
+    # 121 / 103 and 91 / 83.
     DENSE_MAX = 128
 
     def _auto(self, kind, inp, out):

@@ -1,8 +1,10 @@
 // Banded solves along one axis of strided 1-3D arrays (FP64 factors,
 // float64 or complex128 right-hand sides).  All band offsets are even, so the
-// even and odd unknowns form two independent chains: one thread per
-// (line, parity) chain, consecutive threads on consecutive lines so every
-// step of the recurrence is a coalesced access across the wave.
+// even and odd unknowns form two independent chains.  The TDMA and Helmholtz
+// solves cut a chain into segments, a thread each (chain_solve_kernel); the
+// diagonal solve takes a thread per element; the others a thread per (line,
+// parity) chain, consecutive threads on consecutive lines so every step of the
+// recurrence is a coalesced access across the wave.
 #include "common.h"
 
 namespace sfa {
@@ -479,18 +481,18 @@ __global__ void poisson_add_kernel(const T* __restrict__ b, T* __restrict__ u, L
 //
 // Measured against a thread per chain (and, for the Helmholtz solve of one long
 // line, a workgroup whose first thread ran both sweeps from LDS): Helmholtz
-// 128 x 128 x 65 complex 47.7 -> 17.4 us (its arrays are 68 MB: 14 us at copy
-// speed), one line of 1024 reals 45.0 -> 5.2 us; TDMA 192 x 96 x 81 complex with
-// shared factors 51.5 -> 17.1 us, 512 x 129 with factors per line, mode 0 in a
-// launch of its own, 194 + 123 -> 7.8 us in one.
+// 128 x 128 x 65 complex 47.3 -> 18.0 us (its arrays are 68 MB: 14 us at copy
+// speed), one line of 1024 reals 44.8 -> 5.5 us; TDMA 192 x 96 x 81 complex with
+// shared factors 40.1 -> 11.1 us, 510 x 129 with factors per line 133 -> 7.4 us
+// (and mode 0 in the same launch: 123 us in one of its own before).
 //
 // The maps' factors are kept as a number times a power of two: a product of
 // multipliers may pass the largest double, or fall below the smallest, where the
 // values themselves, row by row, stay in range (and a line of zeros stays zero).
 // A segment's factor is split once, after its rows (at most 8 multipliers); the
 // numbers of products over the at most 256 segments then stay far inside the
-// range.  Against plain doubles a solve of few lines takes 0.3 us (TDMA) and 0.9 us
-// (Helmholtz) more, one bound by its bytes the same.
+// range.  Against plain doubles a solve takes 0.3 us (TDMA) and 0.9 to 1.3 us
+// (Helmholtz: 128 x 128 x 65 16.7 -> 18.0) more.
 struct ChainFac {
     double a;
     int e;  // times 2^e

@@ -107,8 +107,9 @@ struct XPassArgs {
 __device__ inline int perm_dct(int i, int N) { return (i & 1) ? (N - 1 - (i >> 1)) : (i >> 1); }
 
 // x-pass without a plan: the factorisation itself as a scan.  With a plan the
-// kernels that start from its restart states take every length up to 514 (218 x
-// 38 x 144: 1042 us here, 160 there; a whole 32^3 solve 23.2 and 21.1 us).
+// kernels that start from its restart states take every length up to 514, past
+// which both forms refuse the solve (218 x 38 x 144: 1042 us here, 160 there; a
+// whole 32^3 solve 23.2 and 20.2 us), for up to 65535 stacked arrays.
 __global__ void __launch_bounds__(256) xpass_kernel(XPassArgs a)
 {
     extern __shared__ double2 smem[];
@@ -414,7 +415,7 @@ static const double* plan_lift(const void* plan)
 
 // The x-pass on the plan's restart states: one kernel for lengths with prime
 // factors up to 13, else a DCT-II, the solve and a DCT-III in place.  False above
-// 514 rows.
+// 514 rows or 65535 arrays.
 static bool xpass_mix(double2* W, int Nx, int Ny, int Nzh, int Kp, double alpha, int neumann, const double* K2,
                       const XPlan& pv, int64_t nb, hipStream_t s, int* rc)
 {

@@ -21,8 +21,7 @@ __device__ inline v4d mfma16(double a, double b, v4d c)
 
 // C (m x n, ldc) = A (m x k, lda) B (k x n, ldb), all row-major FP64, by the
 // whole workgroup (4 waves in a 2 x 2 grid over a BM x BN block tile, K in
-// steps of BK).  sA: BK x (BM + 8), sB: BK x (BN + 8) doubles of LDS (see
-// FoldShape for the pitches).
+// steps of BK).  sA: BK x (BM + 8), sB: BK x (BN + 8) doubles of LDS.
 // Out-of-range operand elements load as zero; stores are bounds-checked.
 // Each output is one MFMA accumulation chain over K in ascending order, so
 // the result does not depend on BM, BN or BK.

@@ -41,8 +41,10 @@ __device__ inline void tile_index(int e, int T, int len, int t_fast, int& t, int
 
 __device__ inline int dct_perm(int i, int N) { return (i & 1) ? (N - 1 - (i >> 1)) : (i >> 1); }
 
-// Lines that neither the in-place passes (factors up to 13) nor Bluestein's
-// algorithm (up to 2048 points) take: a larger prime factor past 2048 points.
+// Lines that neither the in-place passes (lengths up to 4096 with factors up to
+// 13, in at most four of them) nor Bluestein's algorithm (up to 2048 points)
+// take: past 2048 points a larger prime factor or five passes (3125), and every
+// length above 4096 that fits the LDS.
 template <int OP, bool INV>
 __global__ void __launch_bounds__(256) line_kernel(LineArgs a)
 {
