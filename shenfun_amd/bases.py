@@ -332,12 +332,16 @@ class _PolyBase(SpectralBase):
 
     # dense per-line contraction: 'recursive' / 'vandermonde' kinds.  parity: 1
     # if M's rows are the basis functions (analysis), 2 if its columns are
-    # (synthesis), on the family's symmetric nodes
+    # (synthesis), on the family's symmetric nodes.  M's shape says how many rows
+    # of inp are read and of out written (the boundary slots may be left out)
     def _matmul(self, inp, out, M, parity):
-        shp, sin = _geom(inp)
-        _, sout = _geom(out)
-        args = (_lib.ptr(inp), _lib.ptr(out), self._dtype_code(inp), inp.dim(), shp, sin, sout,
-                self.axis, int(M.shape[0]), _lib.ptr(M))
+        nout, nin = M.shape
+        shp = inp.shape
+        if shp[self.axis] != nin:
+            shp = list(shp)
+            shp[self.axis] = nin
+        args = (_lib.ptr(inp), _lib.ptr(out), self._dtype_code(inp), len(shp), _lib.arr(shp),
+                _lib.arr(inp.stride()), _lib.arr(out.stride()), self.axis, nout, _lib.ptr(M))
         if self._even_odd:
             _lib.call("sfa_line_matmul_parity", *args, parity, _lib.stream_ptr())
         else:
@@ -372,10 +376,6 @@ class _PolyBase(SpectralBase):
             torch.cuda.current_stream(M.device).synchronize()  # other streams may take it from the cache
             self._cache[key] = M
         return self._cache[key]
-
-    def _own(self, t):
-        """The rows of this space's own functions (all but the boundary slots)."""
-        return t.narrow(self.axis, 0, self.dim())
 
     # ------------------------------------------------------------ transforms
     def _clone(self, N, padding_factor=1, dealias_direct=False):
@@ -594,7 +594,7 @@ class _PolyBase(SpectralBase):
             # (spectralbase.py:225-229, _truncation_forward :1362-1366)
             twin = self._twin()
             if self._padded_dense(twin, kind, inp, out):  # the kept rows of its matrix, in one product
-                self._matmul(inp, self._own(out), self._padded_matrix("a", twin), 1)
+                self._matmul(inp, out, self._padded_matrix("a", twin), 1)
                 if slots and self.dim() < self.N:
                     out.narrow(self.axis, self.dim(), self.N - self.dim()).zero_()
                 return out
@@ -622,7 +622,7 @@ class _PolyBase(SpectralBase):
             # padded-length synthesis
             twin = self._twin()
             if self._padded_dense(twin, kind, inp, out):
-                self._matmul(self._own(inp), out, self._padded_matrix("s", twin), 2)
+                self._matmul(inp, out, self._padded_matrix("s", twin), 2)
             else:
                 shp = list(inp.shape)
                 shp[self.axis] = self._phys_len()

@@ -135,12 +135,10 @@ class _Banded:
     # solves go through the static Solve resolved by the backend dispatch
     _dispatch = True
 
-    @classmethod
-    def _hip_solve(cls):
+    def _hip_solve(self):
         """Whether Solve resolves to the HIP backend's own function, which a
         launch that does more at once may stand for."""
-        f = getattr(getattr(cls, "Solve", None), "resolved", None)
-        return f is not None and f.__module__ == _HIP
+        return getattr(self.Solve, "backend", None) == _HIP
 
     def __call__(self, b, u=None, axis=0, constraints=()):
         u = _prepare(b, u)

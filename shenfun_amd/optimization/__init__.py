@@ -46,7 +46,7 @@ def optimizer(func, wrap=True):
     @wraps(func)
     def wrapped_function(*args, **kwargs):
         return fun(*args, **kwargs)
-    wrapped_function.resolved = fun
+    wrapped_function.backend = mod.__name__ if fun is not func else None
     return wrapped_function
 
 
