@@ -841,13 +841,17 @@ static void chain_launch_tl(const ChainArgs<T>& a, hipStream_t s)
 //   line per workgroup 300/518, a thread per chain 33/73; 254 x 32768 103/247,
 //   306/520, 146/403; 510 x 131072 938/2193, 1228/2232, 2731/7762); up to 128 of
 //   them are spread over the chip instead (254 x 16: 4.2/5.9 against 4.8/6.3).
-static int chain_tl(int K, int64_t nlines, bool across, bool cplx)
+//   TDMA factors of each line's own lie along memory whatever the lines do, so
+//   those stay at 16 lines where 64 would do (64 x 32768 side by side 27, 64 lines
+//   36) and take a line along memory alone from 193 rows of a chain on (512 x 32768
+//   373, 4 lines 559; up to there 256 x 32768 182, alone 302).
+static int chain_tl(int K, int64_t nlines, bool across, bool cplx, bool own)
 {
-    const int least = K <= 8 ? 64 : K <= 32 ? 16 : K <= 64 ? 8 : K <= 256 ? 4 : 1;
+    const int least = K <= 8 ? 64 : K <= 32 ? 16 : K <= 64 ? 8 : K <= (own ? 192 : 256) ? 4 : 1;
     if (!across) return K > 32 && nlines <= 128 ? 1 : least;
     if (K > 128 && nlines >= 65536) return 64;
     if (K > 256) return nlines < 128 ? 1 : nlines < 2048 ? 4 : 16;
-    const int most = K <= 32 ? 64 : K <= 128 || !cplx ? 16 : 8;
+    const int most = K <= 32 && !own ? 64 : K <= 128 || !cplx ? 16 : 8;
     const int fill = nlines >= 8192 ? 64 : nlines >= 2048 ? 16 : nlines >= 1024 ? 8 : 4;
     const int tl = fill < most ? fill : most;
     return tl > least ? tl : least;
@@ -858,7 +862,7 @@ static void chain_launch(const ChainArgs<T>& a, hipStream_t s)
 {
     auto absl = [](int64_t v) { return v < 0 ? -v : v; };
     const bool across = absl(a.gu.s2) < absl(a.gu.sa) && a.gu.d2 > 1;
-    switch (chain_tl((a.n + 1) / 2, a.gu.nlines, across, sizeof(T) == 16)) {
+    switch (chain_tl((a.n + 1) / 2, a.gu.nlines, across, sizeof(T) == 16, !HELM && a.dls > 0)) {
         case 64: return chain_launch_tl<64, HELM>(a, s);
         case 16: return chain_launch_tl<16, HELM>(a, s);
         case 8: return chain_launch_tl<8, HELM>(a, s);

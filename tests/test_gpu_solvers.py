@@ -474,3 +474,29 @@ def test_chain_scan_lines_per_workgroup(sfa, N, lines, axis, cplx):
         assert float((got[:n] - r[:, idx]).abs().amax()) < TOL * float(r.abs().max())
         if kind == "tdma":
             assert not bool(got[n:].any())
+
+
+@pytest.mark.parametrize("N,lines,axis", [(34, 8201, 0), (35, 8200, 0), (386, 1100, 0), (388, 300, 0),
+                                          (66, 2050, 1), (386, 300, 1), (388, 300, 1), (514, 300, 1)])
+def test_chain_scan_own_factors(sfa, N, lines, axis):
+    """TDMA factors of each line's own where the lines per workgroup depend on
+    it (chains of 16, 17, 192, 193 and 256 rows), vs the oracle's solve with one
+    set, each line's matrix a multiple of it."""
+    print(f"[chain own factors N={N} lines={lines} axis={axis}]", flush=True)
+    from shenfun_amd import _lib
+    rng = np.random.default_rng(N)
+    n = N - 2
+    b = rng.standard_normal((32, N)) + 1j * rng.standard_normal((32, N))
+    d3 = {0: rng.uniform(2, 3, n), -2: rng.uniform(0.1, 1, n - 2), 2: rng.uniform(0.1, 1, n - 2)}
+    dia = S.tdma_dia(d3, n)
+    ref = dev(S.tdma_solve(b[:, :n], S.tdma_lu(dia.copy()), 1))
+    sc = dev(rng.uniform(0.5, 2.0, lines))
+    data = sc[:, None, None] * dev(dia)[None]
+    _lib.call("sfa_tdma_lu", _lib.ptr(data), n, lines, _lib.stream_ptr())
+    idx = torch.arange(lines, device="cuda") % 32
+    u = dev(b)[idx].contiguous() if axis == 1 else dev(b)[idx].T.contiguous()
+    _lib.call("sfa_tdma_solve", _lib.ptr(u), _lib.C128, 2, _lib.arr(u.shape), _lib.arr(u.stride()), axis,
+              _lib.ptr(data), n, 3 * n, 0, _lib.stream_ptr())
+    got = (u if axis == 1 else u.T)[:, :n]
+    want = ref[idx] / sc[:, None]
+    assert float((got - want).abs().amax()) < TOL * float(want.abs().max())
